@@ -356,23 +356,24 @@ __device__ __forceinline__ void nrc_mlp_body(const MlpArgs& a, __bf16* W) {
                 float w[8];
                 level_corners(a.v, l, e.p, idx, w);
                 for (int k = 0; k < 8; ++k) {
-                    float c0 = w[k] * g0, c1 = w[k] * g1;
+                    const float c0 = w[k] * g0, c1 = w[k] * g1;
                     const uint32_t li = (uint32_t)__shfl((int)idx[k], lead);
                     // an invalid lane contributes zero wherever it is counted
                     const uint64_t same = __ballot(!valid || idx[k] == li);
                     const bool merged = ((same >> lead) & 0xFFFFull) == 0xFFFFull;
+                    float m0 = c0, m1 = c1;
                     if (__ballot(merged)) {  // some group of the wave merges: every lane takes part in the sums
                         for (int off = 8; off >= 1; off >>= 1) {
-                            c0 += __shfl_xor(c0, off);
-                            c1 += __shfl_xor(c1, off);
+                            m0 += __shfl_xor(m0, off);
+                            m1 += __shfl_xor(m1, off);
                         }
                     }
                     if (merged) {
                         if (lane == lead && valid) {  // an invalid leader: the whole tile is past the count
-                            unsafeAtomicAdd(a.grid_grad + 2 * (size_t)li, c0);
-                            unsafeAtomicAdd(a.grid_grad + 2 * (size_t)li + 1, c1);
+                            unsafeAtomicAdd(a.grid_grad + 2 * (size_t)li, m0);
+                            unsafeAtomicAdd(a.grid_grad + 2 * (size_t)li + 1, m1);
                         }
-                    } else if (valid) {
+                    } else if (valid) {  // (its own term: the other groups' sums are not its)
                         unsafeAtomicAdd(a.grid_grad + 2 * (size_t)idx[k], c0);
                         unsafeAtomicAdd(a.grid_grad + 2 * (size_t)idx[k] + 1, c1);
                     }
