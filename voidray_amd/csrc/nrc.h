@@ -60,6 +60,8 @@ struct vr_cache {
     // training scratch: transposed inputs/activations/deltas, split-K partials
     uint32_t train_cap = 0;
     __bf16 *xT = nullptr, *hT = nullptr, *dT = nullptr;
+    float* gx = nullptr;         // [level][train_cap][2] gradients of the grid features
+    uint32_t* gslice = nullptr;  // [level][train_cap] table slices a sample touches (k_nrc_scatter)
     float* part = nullptr;
     float* loss = nullptr;       // [0] sum of loss terms, [1] mean loss of the last step
     uint32_t* counts = nullptr;

@@ -209,6 +209,8 @@ struct MlpArgs {
     __bf16 *xT, *hT, *dT; // training: transposed [rows][cap]
     uint32_t cap;
     float* grid_grad;
+    float* gx;            // training: [level][cap][2] gradients of the grid features for k_nrc_scatter
+    uint32_t* gslice;     // training: [level][cap] the slices of a hashed level's four (y, z) corner pairs
     uint32_t part, parts;  // training mini-batch: slice part of parts of the samples
 };
 
@@ -234,10 +236,54 @@ __device__ __forceinline__ void load_weights(const __bf16* src, __bf16* W) {
     }
 }
 
+// The grid-gradient scatter cuts a level's table into slices of 2^14 entries.
+constexpr int kScatLog = 14, kScatSlice = 1 << kScatLog;
+// Both entries of a corner pair (x and x + 1 at one (y, z)) fall into one
+// slice: a hashed level's slice is (y p1 ^ z p2) >> 14 while x stays below 2^14
+// (scat_by_yz), and a dense level's slices are whole rows of x.
+struct ScatLevel {
+    uint32_t rows;    // dense: rows (y, z) per slice; 0: hashed
+    float inv_rows;
+    uint32_t slices, len;  // slices of the level, entries of a slice
+};
+__host__ __device__ inline ScatLevel scat_level(const NrcView& v, int l) {
+    ScatLevel s;
+    const uint32_t table = v.table_mask + 1u, w = v.res[l] + 1u;
+    if (v.dense[l] && w <= (uint32_t)kScatSlice) {
+        s.rows = (uint32_t)kScatSlice / w;
+        s.inv_rows = 1.0f / (float)s.rows;
+        s.slices = (w * w + s.rows - 1u) / s.rows;
+        s.len = s.rows * w;
+    } else {
+        s.rows = 0;
+        s.inv_rows = 0.f;
+        s.slices = (table + kScatSlice - 1u) / kScatSlice;
+        s.len = kScatSlice;
+    }
+    return s;
+}
+__device__ __forceinline__ bool scat_by_yz(const NrcView& v, int l) { return v.dense[l] || v.res[l] < (uint32_t)kScatSlice; }
+// The slices of the corner pairs (y + bit 0, z + bit 1), a byte each.  (Row
+// numbers stay below 2^16 and quotients below 2^10, so the product with the
+// reciprocal, half a row up, truncates to the quotient.)
+__device__ __forceinline__ uint32_t scat_slices(const NrcView& v, int l, const ScatLevel& s, uint32_t y, uint32_t z) {
+    const uint32_t w = v.res[l] + 1u;
+    uint32_t ids = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t yk = y + (k & 1), zk = z + (k >> 1);
+        const uint32_t id = s.rows ? (uint32_t)(((float)(yk + w * zk) + 0.5f) * s.inv_rows)
+                                   : ((yk * 2654435761u ^ zk * 805459861u) & v.table_mask) >> kScatLog;
+        ids |= id << (8 * k);
+    }
+    return ids;
+}
+
 // Fused encode + MLP forward (+ loss, backward, grid scatter, transposed
 // stores for the weight gradients when TRAIN).  One wave = 16 samples per
 // iteration; all 64 lanes take part in every MFMA.
-template <bool TRAIN>
+// SCATTER: the grid gradients are left to k_nrc_scatter.
+template <bool TRAIN, bool SCATTER = false>
 __device__ __forceinline__ void nrc_mlp_body(const MlpArgs& a, __bf16* W) {
     load_weights(a.v.w_bf, W);
     __syncthreads();
@@ -347,6 +393,20 @@ __device__ __forceinline__ void nrc_mlp_body(const MlpArgs& a, __bf16* W) {
         // same-address atomics.
         f32x4 dx[2];
         bwd_hidden(W + kL0, kS0, 2, d0, dx, col, q);
+        if (SCATTER) {
+            for (int t = 0; t < 2; ++t)
+                for (int lv = 0; lv < 2; ++lv)
+                {
+                    const int l = 8 * t + 2 * q + lv;
+                    ((float2*)a.gx)[(size_t)l * cs + s] = make_float2(dx[t][2 * lv], dx[t][2 * lv + 1]);
+                    if (!scat_by_yz(a.v, l)) continue;
+                    const uint32_t r = a.v.res[l];  // as level_corners
+                    const uint32_t y = min((uint32_t)floorf(e.p[1] * (float)r), r - 1);
+                    const uint32_t z = min((uint32_t)floorf(e.p[2] * (float)r), r - 1);
+                    a.gslice[(size_t)l * cs + s] = scat_slices(a.v, l, scat_level(a.v, l), y, z);
+                }
+            continue;
+        }
         const int lead = lane & ~15;
         for (int t = 0; t < 2; ++t)
             for (int lv = 0; lv < 2; ++lv) {
@@ -388,9 +448,154 @@ __global__ __launch_bounds__(kFwdBlock, 2) void k_nrc_infer(MlpArgs a) {
     __shared__ __attribute__((aligned(16))) __bf16 W[kLdsW];
     nrc_mlp_body<false>(a, W);
 }
+template <bool SCATTER>
 __global__ __launch_bounds__(kFwdBlock) void k_nrc_train(MlpArgs a) {
     __shared__ __attribute__((aligned(16))) __bf16 W[kLdsW];
-    nrc_mlp_body<true>(a, W);
+    nrc_mlp_body<true, SCATTER>(a, W);
+}
+
+// Grid gradients: sums, over the samples, of weight x feature gradient into
+// the 8 entries a sample touches per level.  Added to memory one by one (the
+// path inside k_nrc_train), each of the 2^24 atomics of a 2^16-sample step goes
+// to the memory side as a write of its own (0.63 GB a step, about 16 G/s: 1.07
+// of the step's 1.36 ms).  Here a block owns a slice of one level's table in
+// LDS, picks the samples that touch it, adds what they give and writes the
+// touched entries once: no atomic leaves the CU.  k_nrc_train has left the
+// slices of a sample's four (y, z) corner pairs in one word per level, so a
+// block passes over a sample with a load and a few instructions; the samples
+// that touch the slice (1 in 8) are queued per wave and worked on 64 at a time.
+// 146 us for 2^16 samples (2^19 entries a level), 48 us for 2^13; with the
+// indices recomputed by every block, lanes without a hit idle, 272 us.
+// Levels with fewer slices than blocks (the dense coarse ones, whose entries
+// many samples share) split the samples among the blocks instead, which then
+// add their slices to memory atomically.
+constexpr int kScatBlock = 1024;
+constexpr uint32_t kScatMinBlocks = 32;  // blocks per level: 512 in all, two rounds of the 256 CUs
+// More slices mean more passes over the samples (and have to fit a byte);
+// few samples are cheaper to add one by one.
+constexpr uint32_t kScatMaxSlices = 64;
+constexpr uint32_t kScatMinSamples = 2048;
+
+
+__global__ __launch_bounds__(kScatBlock) void k_nrc_scatter(NrcView v, const float* pos, const float* gx,
+                                                            const uint32_t* gslice, uint32_t cap, const uint32_t* d_n,
+                                                            uint32_t n_host, uint32_t mb, uint32_t mbs,
+                                                            uint32_t level_blocks, float* grid_grad) {
+    __shared__ __attribute__((aligned(16))) float acc[2 * kScatSlice];
+    __shared__ u32x2 queue[kScatBlock / 64][128];  // per wave: (sample, bit 8k + 7: corner pair k)
+    uint32_t begin = 0, n = 0;
+    slice_of(d_n ? min(*d_n, n_host) : n_host, mb, mbs, begin, n);
+    // workgroups are dealt round-robin to the 8 XCDs: a level's blocks share
+    // one XCD's L2, where its samples' words stay
+    const int level = (int)((blockIdx.x & 7u) | ((blockIdx.x >> 3) & 1u) << 3);
+    const uint32_t j = blockIdx.x >> 4, table = v.table_mask + 1u, r = v.res[level];  // j < level_blocks
+    const bool dense = v.dense[level] != 0;
+    const uint32_t entries = dense ? (r + 1) * (r + 1) * (r + 1) : table;
+    const ScatLevel sl = scat_level(v, level);
+    const uint32_t slices = sl.slices, chunks = level_blocks / slices;
+    const uint32_t slice = j % slices, chunk = j / slices;
+    if (chunk >= chunks) return;
+    const uint32_t lo = slice * sl.len, len = min(sl.len, entries - lo);
+    for (uint32_t i = threadIdx.x; i < (len + 1) / 2; i += kScatBlock) ((f32x4*)acc)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+    const uint32_t s0 = (uint32_t)((uint64_t)n * chunk / chunks), s1 = (uint32_t)((uint64_t)n * (chunk + 1) / chunks);
+    const float* p = pos + 3 * (size_t)begin;
+    const float2* g = (const float2*)gx + (size_t)level * cap;
+    const float fr = (float)r;
+    const uint32_t ym = dense ? r + 1 : 2654435761u, zm = dense ? (r + 1) * (r + 1) : 805459861u;
+    uint32_t c[3];
+    float f[3];
+    float2 gs;
+    auto load = [&](uint32_t s) {  // cell and offsets as level_corners
+        for (int a = 0; a < 3; ++a) {
+            const float x = clamp01((p[3 * (size_t)s + a] - v.origin[a]) * v.inv_extent) * fr;
+            uint32_t ci = (uint32_t)floorf(x);
+            if (ci > r - 1) ci = r - 1;
+            c[a] = ci;
+            f[a] = x - (float)ci;
+        }
+        gs = g[s];
+    };
+    // corner k: (cx + bit 0, cy + bit 1, cz + bit 2)
+    auto index = [&](uint32_t k) {
+        const uint32_t x = c[0] + (k & 1u), y = c[1] * ym + (k & 2u ? ym : 0u), z = c[2] * zm + (k & 4u ? zm : 0u);
+        return dense ? x + y + z : (x ^ y ^ z) & v.table_mask;
+    };
+    auto add = [&](uint32_t k, uint32_t i) {
+        const float wx = (k & 1u) ? f[0] : 1.f - f[0], wy = (k & 2u) ? f[1] : 1.f - f[1],
+                    wz = (k & 4u) ? f[2] : 1.f - f[2];
+        const float w = (wx * wy) * wz;
+        unsafeAtomicAdd(&acc[2 * i], w * gs.x);
+        unsafeAtomicAdd(&acc[2 * i + 1], w * gs.y);
+    };
+    if (slices > 1 && scat_by_yz(v, level)) {
+        const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+        const uint32_t* ids = gslice + (size_t)level * cap;
+        u32x2* q = queue[wave];
+        auto work = [&](u32x2 e) {
+            load(e.x);
+            for (uint32_t m = e.y; m; m &= m - 1u) {
+                const uint32_t k = ((uint32_t)__builtin_ctz(m) >> 3) << 1;
+                add(k, index(k) - lo);
+                add(k | 1u, index(k | 1u) - lo);
+            }
+        };
+        // four samples a lane and load, four loads in flight
+        constexpr int kAhead = 4;
+        const uint32_t none = 0xFFFFFFFFu;  // (no slice is 255)
+        uint32_t cnt = 0;                   // queued (wave-uniform, < 64 between the steps)
+        for (uint32_t sb = (s0 & ~3u) + 256u * wave; sb < s1; sb += kAhead * 4 * kScatBlock) {
+            u32x4 id[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const uint32_t s = sb + u * 4 * kScatBlock + 4u * lane;
+                id[u] = s < s1 ? *(const u32x4*)(ids + s) : u32x4{none, none, none, none};
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t s = sb + u * 4 * kScatBlock + 4u * lane + (uint32_t)i;
+                    const uint32_t x = (i == 0 ? id[u].x : i == 1 ? id[u].y : i == 2 ? id[u].z : id[u].w) ^
+                                       (slice * 0x01010101u);
+                    uint32_t hit = ~(((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x | 0x7F7F7F7Fu);  // 0x80 in every zero byte
+                    if (s < s0 || s >= s1) hit = 0;
+                    const uint64_t m = __ballot(hit != 0u);
+                    if (m == 0ull) continue;
+                    if (hit) q[cnt + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = u32x2{s, hit};
+                    cnt += (uint32_t)__popcll(m);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    if (cnt >= 64u) {
+                        cnt -= 64u;
+                        work(q[cnt + lane]);
+                        __builtin_amdgcn_wave_barrier();  // read before the next step writes
+                    }
+                }
+            }
+        }
+        if (lane < cnt) work(q[lane]);
+    } else {
+        for (uint32_t s = s0 + threadIdx.x; s < s1; s += kScatBlock) {
+            load(s);
+            for (uint32_t k = 0; k < 8; ++k) {
+                const uint32_t i = index(k) - lo;
+                if (i < len) add(k, i);
+            }
+        }
+    }
+    __syncthreads();
+    float2* out = (float2*)grid_grad + ((size_t)level << v.log2_table) + lo;
+    for (uint32_t i = threadIdx.x; i < len; i += kScatBlock) {
+        const float2 x = ((const float2*)acc)[i];
+        if (x.x == 0.f && x.y == 0.f) continue;
+        if (chunks > 1) {
+            unsafeAtomicAdd(&out[i].x, x.x);
+            unsafeAtomicAdd(&out[i].y, x.y);
+        } else {
+            out[i] = x;  // this block's alone, and zero before (nrc_train_step)
+        }
+    }
 }
 
 // dW_L = sum over samples of delta_L (x) input_L, split over blocks along the
@@ -681,11 +886,17 @@ int ensure_train_scratch(vr_cache* c, uint32_t n) {
     if (c->xT) VR_HIP_CHECK(hipFree(c->xT));
     if (c->hT) VR_HIP_CHECK(hipFree(c->hT));
     if (c->dT) VR_HIP_CHECK(hipFree(c->dT));
+    if (c->gx) VR_HIP_CHECK(hipFree(c->gx));
+    if (c->gslice) VR_HIP_CHECK(hipFree(c->gslice));
     c->xT = c->hT = c->dT = nullptr;
+    c->gx = nullptr;
+    c->gslice = nullptr;
     c->train_cap = 0;
     if (hipMalloc((void**)&c->xT, (size_t)kNrcIn * need * 2) != hipSuccess ||
         hipMalloc((void**)&c->hT, (size_t)4 * kNrcHid * need * 2) != hipSuccess ||
-        hipMalloc((void**)&c->dT, (size_t)(4 * kNrcHid + kNrcOut) * need * 2) != hipSuccess)
+        hipMalloc((void**)&c->dT, (size_t)(4 * kNrcHid + kNrcOut) * need * 2) != hipSuccess ||
+        hipMalloc((void**)&c->gx, (size_t)2 * kNrcLevels * need * 4) != hipSuccess ||
+        hipMalloc((void**)&c->gslice, (size_t)kNrcLevels * need * 4) != hipSuccess)
         return fail(VR_ERR_OOM, "radiance cache training scratch allocation failed");
     c->train_cap = need;
     return 0;
@@ -702,6 +913,14 @@ MlpArgs make_args(vr_cache* c, uint32_t n, const uint32_t* d_n, const float* pos
     a.nrm = nrm;
     a.rough = rough;
     return a;
+}
+
+// Blocks per level of k_nrc_scatter: one per slice of the level that has the
+// most, and no less than kScatMinBlocks.
+uint32_t scat_level_blocks(const vr_cache* c) {
+    uint32_t m = kScatMinBlocks;
+    for (int l = 0; l < kNrcLevels; ++l) m = std::max(m, scat_level(c->view, l).slices);
+    return m;
 }
 
 uint32_t mlp_blocks(uint32_t n) {
@@ -746,7 +965,16 @@ int nrc_train_step(vr_cache* c, uint32_t n, const uint32_t* d_n, const float* po
             a.dT = c->dT;
             a.cap = c->train_cap;
             // a mini-batch holds at most ceil(n / parts) samples: no blocks beyond those
-            hipLaunchKernelGGL(k_nrc_train, dim3(mlp_blocks((n + parts - 1) / parts)), dim3(kFwdBlock), 0, st, a);
+            a.gx = c->gx;
+            a.gslice = c->gslice;
+            const uint32_t n_part = (n + parts - 1) / parts, level_blocks = scat_level_blocks(c);
+            const bool scatter = n_part >= kScatMinSamples && level_blocks <= kScatMaxSlices;
+            void (*train)(MlpArgs) = scatter ? k_nrc_train<true> : k_nrc_train<false>;
+            hipLaunchKernelGGL(train, dim3(mlp_blocks(n_part)), dim3(kFwdBlock), 0, st, a);
+            if (scatter)
+                hipLaunchKernelGGL(k_nrc_scatter, dim3(kNrcLevels * level_blocks), dim3(kScatBlock), 0, st, c->view, pos,
+                                   (const float*)c->gx, (const uint32_t*)c->gslice, c->train_cap, d_n, n, part, parts,
+                                   level_blocks, c->g_grad);
             hipLaunchKernelGGL(k_nrc_wgrad, dim3(kWgradBlocks, 5), dim3(256), 0, st, (const __bf16*)c->xT,
                                (const __bf16*)c->hT, (const __bf16*)c->dT, c->train_cap, d_n, n, part, parts,
                                c->part);
@@ -849,7 +1077,7 @@ int nrc_order_samples(vr_cache* c, uint32_t parts, uint32_t frame, hipStream_t s
 // ---------------------------------------------------------------------------
 static void free_cache(vr_cache* c) {
     void* ptrs[] = {c->w_master, c->w_m, c->w_v, c->w_grad, c->w_bf, c->g_master, c->g_m, c->g_v, c->g_grad, c->g_h,
-                    c->xT, c->hT, c->dT, c->part, c->loss, c->counts};
+                    c->xT, c->hT, c->dT, c->gx, c->gslice, c->part, c->loss, c->counts};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (void* p : c->frame_allocs) (void)hipFree(p);
