@@ -196,7 +196,7 @@ int vr_trace_host(const vr_scene_desc* sd, const vr_trace_desc* desc, const floa
         const bool any = mode == VR_TRACE_ANY;
         constexpr int kStack = 16, kSpill = 240;
         u32x2 lds[kStack], spill[kSpill];
-        const vr::WideStack ws{lds, 1, spill, 1, kSpill};
+        const vr::WideStack ws{(vr::lds_u32x2*)lds, 1, spill, 1, kSpill};
         uint32_t fb = 0;
         for (uint32_t i = 0; i < n; ++i) {
             const vf3 oi = mk3(o[3 * i], o[3 * i + 1], o[3 * i + 2]), di = mk3(d[3 * i], d[3 * i + 1], d[3 * i + 2]);

@@ -7,7 +7,7 @@
 //    reference engine walks it for the rare rays whose closest hit cannot be
 //    confirmed that way.
 //  * build_qbvh: a binned-SAH binary BVH with spatial splits collapsed to
-//    4-wide nodes with 8-bit outward-rounded child boxes (QNode, 64 B) and
+//    8-wide nodes with 8-bit outward-rounded child boxes (QNode, 80 B) and
 //    triangle records in leaf order.
 #include <algorithm>
 #include <atomic>
@@ -554,6 +554,68 @@ static int pick_exponent(float lo, float hi) {
     return std::max(e, -100);
 }
 
+// Which binary nodes become the children of the wide nodes: the cut of least
+// SAH cost, by dynamic programming over the binary tree (Ylitie, Karras &
+// Laine 2017, section 4.1).  cost[8 n + i - 1]: least cost of node n's subtree
+// as at most i children; split[8 n + i - 1]: how many of them its left child
+// gets, 0: as with i - 1 (i = 1: n is one child, a leaf or a wide node).
+struct Collapse {
+    static constexpr float kNode = 1.0f, kTri = 0.35f;  // a record test costs about a third of a node visit
+    const std::vector<BNode>& bn;
+    std::vector<float> cost;
+    std::vector<uint8_t> split;
+
+    explicit Collapse(const std::vector<BNode>& b) : bn(b), cost(8 * b.size()), split(8 * b.size()) {
+        for (size_t n = b.size(); n-- > 0;) {  // pre-order: children come after their parent
+            float* c = &cost[8 * n];
+            uint8_t* s = &split[8 * n];
+            const float area = b[n].box.area();
+            if (b[n].child[0] < 0) {
+                for (int i = 0; i < 8; ++i) {
+                    c[i] = area * kTri * (float)b[n].count;
+                    s[i] = 0;
+                }
+                continue;
+            }
+            const float* l = &cost[8 * (size_t)b[n].child[0]];
+            const float* r = &cost[8 * (size_t)b[n].child[1]];
+            float best8 = kInf;
+            for (int i = 2; i <= 8; ++i) {
+                float best = kInf;
+                int at = 1;
+                for (int k = 1; k < i; ++k)
+                    if (l[k - 1] + r[i - k - 1] < best) {
+                        best = l[k - 1] + r[i - k - 1];
+                        at = k;
+                    }
+                c[i - 1] = best;
+                s[i - 1] = (uint8_t)at;
+                best8 = best;
+            }
+            c[0] = best8 + area * kNode;
+            s[0] = s[7];  // one child: a wide node, whose own children are the cut of 8
+            for (int i = 2; i <= 8; ++i)
+                if (c[i - 2] <= c[i - 1]) {
+                    c[i - 1] = c[i - 2];
+                    s[i - 1] = 0;
+                }
+        }
+    }
+    // The children of node n in a cut of at most i (i >= 2), appended to kids.
+    void children(int32_t n, int i, int32_t* kids, int& nk) const {
+        while (i > 1 && split[8 * (size_t)n + i - 1] == 0) --i;
+        if (i == 1 || bn[n].child[0] < 0) {
+            kids[nk++] = n;
+            return;
+        }
+        open(n, split[8 * (size_t)n + i - 1], i, kids, nk);
+    }
+    void open(int32_t n, int k, int i, int32_t* kids, int& nk) const {
+        children(bn[n].child[0], k, kids, nk);
+        children(bn[n].child[1], i - k, kids, nk);
+    }
+};
+
 }  // namespace
 
 int build_qbvh(const std::vector<TriRec>& tris_in, std::vector<QNode>& qnodes, std::vector<TriRec>& tris_out,
@@ -564,7 +626,7 @@ int build_qbvh(const std::vector<TriRec>& tris_in, std::vector<QNode>& qnodes, s
     depth_out = 0;
     if (n == 0) return 0;
     if (n >= (1u << 27)) {
-        err = "too many triangles for the 27-bit leaf encoding";
+        err = "too many triangles for the 27-bit record indices";
         return -1;
     }
     // references: every triangle with its padded box
@@ -616,71 +678,74 @@ int build_qbvh(const std::vector<TriRec>& tris_in, std::vector<QNode>& qnodes, s
         }
     }
     if (order.size() >= (1u << 27)) {
-        err = "too many triangle references for the 27-bit leaf encoding";
+        err = "too many triangle references for the 27-bit record indices";
         return -1;
     }
     const int32_t root = 0;
-    tris_out.resize(order.size());
-    for (size_t i = 0; i < order.size(); ++i) tris_out[i] = tris_in[order[i]];
 
-    // collapse to 4-wide: children of a wide node = up to 4 binary nodes
+    // collapse to 8-wide: children of a wide node = up to 8 binary nodes
     struct Pending {
         int32_t bnode;
         uint32_t qindex;
         uint32_t depth;
     };
     std::vector<Pending> work;
-    qnodes.reserve(n / 2 + 1);
+    qnodes.reserve(n / 4 + 1);
+    tris_out.reserve(order.size());
     auto is_leaf = [&](int32_t b) { return bn[b].child[0] < 0; };
-    auto leaf_code = [&](int32_t b) -> uint32_t {
-        return kLeafBit | ((bn[b].count - 1) << 27) | bn[b].start;
-    };
+    const Collapse cut(bn);
     // A leaf-only tree gets a single wide node with one leaf child.
     qnodes.push_back(QNode{});
     work.push_back({root, 0, 1});
-    size_t wi = 0;
-    while (wi < work.size()) {
-        Pending pw = work[wi++];
+    while (!work.empty()) {
+        const Pending pw = work.back();  // depth first: a subtree's nodes and records stay close together
+        work.pop_back();
         depth_out = std::max(depth_out, pw.depth);
-        int32_t kids[4];
+        int32_t kids[8];
         int nk = 0;
-        if (is_leaf(pw.bnode)) {
-            kids[nk++] = pw.bnode;
-        } else {
-            kids[nk++] = bn[pw.bnode].child[0];
-            kids[nk++] = bn[pw.bnode].child[1];
-            while (nk < 4) {
-                // open the internal child with the largest surface area
-                int best = -1;
-                float ba = -1.f;
-                for (int i = 0; i < nk; ++i)
-                    if (!is_leaf(kids[i]) && bn[kids[i]].box.area() > ba) {
-                        ba = bn[kids[i]].box.area();
-                        best = i;
-                    }
-                if (best < 0) break;
-                int32_t b = kids[best];
-                kids[best] = bn[b].child[0];
-                kids[nk++] = bn[b].child[1];
-            }
-        }
-        // quantise
+        if (is_leaf(pw.bnode)) kids[nk++] = pw.bnode;
+        else cut.open(pw.bnode, cut.split[8 * (size_t)pw.bnode], 8, kids, nk);
         BBox nb;
         nb.empty();
         for (int i = 0; i < nk; ++i) nb.grow(bn[kids[i]].box);
+        // inner children first, each kind ascending along the axis on which the centres spread most
+        auto centre = [&](int32_t k, int a) { return bn[k].box.lo[a] + bn[k].box.hi[a]; };
+        int axis = 0;
+        float spread = -1.f;
+        for (int a = 0; a < 3; ++a) {
+            float lo = kInf, hi = -kInf;
+            for (int i = 0; i < nk; ++i) {
+                lo = std::min(lo, centre(kids[i], a));
+                hi = std::max(hi, centre(kids[i], a));
+            }
+            if (hi - lo > spread) {
+                spread = hi - lo;
+                axis = a;
+            }
+        }
+        for (int i = 1; i < nk; ++i)
+            for (int k = i; k > 0; --k) {
+                const bool li = is_leaf(kids[k - 1]), lk = is_leaf(kids[k]);
+                if (!(li && !lk) && !(li == lk && centre(kids[k], axis) < centre(kids[k - 1], axis))) break;
+                std::swap(kids[k], kids[k - 1]);
+            }
         QNode q{};
         q.ox = nb.lo[0];
         q.oy = nb.lo[1];
         q.oz = nb.lo[2];
-        q.nchild = (uint8_t)nk;
-        float org[3] = {nb.lo[0], nb.lo[1], nb.lo[2]};
+        const float org[3] = {nb.lo[0], nb.lo[1], nb.lo[2]};
         uint8_t ex[3];
         for (int a = 0; a < 3; ++a) {
             int e = pick_exponent(nb.lo[a], nb.hi[a]);
             for (;;) {
                 bool ok = true;
                 double s = std::ldexp(1.0, e);
-                for (int i = 0; i < nk && ok; ++i) {
+                for (int i = 0; i < 8 && ok; ++i) {
+                    if (i >= nk) {
+                        q.qlo[a][i] = 255;
+                        q.qhi[a][i] = 0;
+                        continue;
+                    }
                     const BBox& cbx = bn[kids[i]].box;
                     double ql = std::floor(((double)cbx.lo[a] - (double)org[a]) / s);
                     double qh = std::ceil(((double)cbx.hi[a] - (double)org[a]) / s);
@@ -703,20 +768,18 @@ int build_qbvh(const std::vector<TriRec>& tris_in, std::vector<QNode>& qnodes, s
         q.ex = ex[0];
         q.ey = ex[1];
         q.ez = ex[2];
-        for (int i = 0; i < 4; ++i) q.child[i] = kInvalidChild;
-        for (int i = nk; i < 4; ++i)
-            for (int a = 0; a < 3; ++a) {
-                q.qlo[a][i] = 255;
-                q.qhi[a][i] = 0;
-            }
+        q.child_base = (uint32_t)qnodes.size();
+        q.tri_base = (uint32_t)tris_out.size();
+        q.leaf_bits = (uint32_t)axis << 24;
         for (int i = 0; i < nk; ++i) {
-            if (is_leaf(kids[i])) {
-                q.child[i] = leaf_code(kids[i]);
+            const int32_t k = kids[i];
+            if (is_leaf(k)) {
+                q.leaf_bits |= ((1u << bn[k].count) - 1u) << (3 * i);
+                for (uint32_t t = 0; t < bn[k].count; ++t) tris_out.push_back(tris_in[order[bn[k].start + t]]);
             } else {
-                uint32_t ci = (uint32_t)qnodes.size();
+                ++q.num_inner;
+                work.push_back({k, (uint32_t)qnodes.size(), pw.depth + 1});
                 qnodes.push_back(QNode{});
-                q.child[i] = ci;
-                work.push_back({kids[i], ci, pw.depth + 1});
             }
         }
         qnodes[pw.qindex] = q;
@@ -725,7 +788,7 @@ int build_qbvh(const std::vector<TriRec>& tris_in, std::vector<QNode>& qnodes, s
             const QNode& w = qnodes[pw.qindex];
             const double wo[3] = {w.ox, w.oy, w.oz};
             const int we[3] = {w.ex, w.ey, w.ez};
-            for (int i = 0; i < nk; ++i)
+            for (int i = 0; i < nk; ++i) {
                 for (int a = 0; a < 3; ++a) {
                     const double s = std::ldexp(1.0, we[a] - 127);
                     const double lo = wo[a] + w.qlo[a][i] * s, hi = wo[a] + w.qhi[a][i] * s;
@@ -733,6 +796,7 @@ int build_qbvh(const std::vector<TriRec>& tris_in, std::vector<QNode>& qnodes, s
                     ++check->boxes_checked;
                     if (!(lo <= (double)ex.lo[a] && hi >= (double)ex.hi[a])) ++check->boxes_not_containing;
                 }
+            }
         }
     }
     return 0;

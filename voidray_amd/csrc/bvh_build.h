@@ -14,7 +14,7 @@ struct QbvhCheck {
     uint64_t boxes_checked = 0;     // (child, axis) pairs
     uint64_t boxes_not_containing = 0;
 };
-// SAH-built 4-wide quantised BVH; tris_out = tris_in in leaf order.
+// SAH-built 8-wide quantised BVH; tris_out = tris_in in leaf order.
 int build_qbvh(const std::vector<TriRec>& tris_in, std::vector<QNode>& qnodes, std::vector<TriRec>& tris_out,
                uint32_t& depth, std::string& err, QbvhCheck* check = nullptr);
 }  // namespace vr

@@ -21,22 +21,30 @@ int fail(int code, const std::string& msg);
             return ::vr::fail(VR_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(_e));           \
     } while (0)
 
-// ---- wide quantised BVH node (64 B, one cache line pair of dwordx4 loads) --
+// ---- wide quantised BVH node: 8 children, 80 B, five dwordx4 loads ----------
 // Child boxes are stored as 8-bit offsets on a per-node, per-axis power-of-two
 // grid anchored at `origin`, rounded outward (lo floored, hi ceiled), so the
-// decoded box always contains the exact (padded) child box.
+// decoded box always contains the exact (padded) child box.  Slots 0 ..
+// num_inner - 1 are inner children, the next ones leaves, both in ascending
+// order of their centres along `axis`.  The inner children are consecutive
+// nodes (slot s is node child_base + s) and the leaves' records consecutive
+// from tri_base on, so a node needs two indices however many children it has
+// (as in the compressed wide BVH of Ylitie, Karras & Laine, HPG 2017).
 struct alignas(16) QNode {
     float ox, oy, oz;
-    uint8_t ex, ey, ez, nchild;  // biased exponents: scale = 2^(e - 127)
-    uint32_t child[4];           // internal: node index; leaf: kLeafBit | (count-1) << 27 | first
-    uint8_t qlo[3][4];           // [axis][child]
-    uint8_t qhi[3][4];
-    uint32_t pad[2];
+    uint8_t ex, ey, ez;          // biased exponents: scale = 2^(e - 127)
+    uint8_t num_inner;
+    uint32_t child_base;         // first inner child
+    uint32_t tri_base;           // first record of the node's leaves
+    uint32_t leaf_bits;          // bits 3s .. 3s + 2: the record count of the leaf in slot s, in unary;
+                                 // bits 24, 25: axis
+    uint32_t pad;
+    uint8_t qlo[3][8];           // [axis][slot]; empty slots: lo 255, hi 0
+    uint8_t qhi[3][8];
 };
-static_assert(sizeof(QNode) == 64, "QNode must be 64 bytes");
-constexpr uint32_t kLeafBit = 0x80000000u;
+static_assert(sizeof(QNode) == 80, "QNode must be 80 bytes");
 constexpr uint32_t kInvalidChild = 0xFFFFFFFFu;
-constexpr uint32_t kMaxLeaf = 3;  // triangles per leaf (count-1 fits 3 bits; 4 measured 0.7% slower)
+constexpr uint32_t kMaxLeaf = 3;  // triangles per leaf (QNode::leaf_bits has 3 bits a slot)
 
 // Triangle record in leaf order (48 B): world-space vertices exactly as the
 // reference stores them and the global prim id.  Prim ids number the

@@ -3,7 +3,7 @@
 // the per-mesh BVH build of Mesh::from_buffers (core/mesh.rs:76-116).
 //
 // HBM layout (all arrays 256-byte aligned, one allocation each):
-//   qnodes   QNode[num_qnodes]      64 B  SAH 4-wide with spatial splits, 8-bit outward-quantised
+//   qnodes   QNode[num_qnodes]      80 B  SAH 8-wide with spatial splits, 8-bit outward-quantised
 //   tris     TriRec[R]              48 B  world vertices in leaf order + prim id (R >= T:
 //                                         one record per leaf holding a piece of a split triangle)
 //   ref/top  RefNode[]              32 B  reference median-split trees (exact engine)
@@ -410,12 +410,11 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
                 if (build_qbvh(brec, bq, bt, bdepth, err, &qcheck) != 0) return fail(VR_ERR_INVALID, err);
                 const uint32_t qoff = (uint32_t)qn.size(), toff = (uint32_t)tris.size();
                 if ((uint64_t)toff + bt.size() >= (1ull << 27))
-                    return fail(VR_ERR_INVALID, "too many triangle references for the 27-bit leaf encoding");
-                for (QNode& q : bq)
-                    for (int c = 0; c < 4; ++c) {
-                        if (q.child[c] == kInvalidChild) continue;
-                        q.child[c] = (q.child[c] & kLeafBit) ? q.child[c] + toff : q.child[c] + qoff;
-                    }
+                    return fail(VR_ERR_INVALID, "too many triangle references for the 27-bit record indices");
+                for (QNode& q : bq) {
+                    q.child_base += qoff;
+                    q.tri_base += toff;
+                }
                 qn.insert(qn.end(), bq.begin(), bq.end());
                 tris.insert(tris.end(), bt.begin(), bt.end());
                 blas_of[x.mesh] = qoff;

@@ -9,20 +9,27 @@
 namespace vr {
 
 constexpr int kWave = 64;        // gfx950 wavefront size; one wave per block
-// LDS stack entries per lane (8 B each): 5 KB per wave, so 32 waves per CU
-// (160 KB of LDS) fit, as many as the closest-hit kernel's 64 VGPRs allow
-// (8 per SIMD).  Measured against 12 entries (6 waves): microbench 0.8%
-// faster, terrain frame 2.4% faster, the cornell room (long bounce chains,
-// deeper stacks) 5% slower; 14 entries 4% slower.
+// LDS stack entries per lane (8 B each).  The tree pushes one entry a level at
+// most and is 9 to 10 levels deep on the million-triangle scenes, so next to
+// nothing spills; 5 and 6 KB per wave allow the 7 waves per SIMD that the
+// registers do.
 constexpr int kLdsStack = 10;
-constexpr int kLdsStackAny = 12;  // any hit: 6, 8, 10 and 11 entries each measured slower (0.4-3.8%)
+constexpr int kLdsStackAny = 12;
 constexpr int kSpillCap = 48;    // global spill entries per lane beyond the LDS part
-constexpr int kRefill = 40;      // idle lanes that trigger a wave-wide refill (closest hit; 24, 32, 48 and 56 measured slower)
-constexpr int kRefillAny = 40;   // the same for any-hit queries (shorter rays: refill less often)
-constexpr int kNodeSteps = 4;    // most node-phase iterations between two leaf phases
+// Idle lanes that trigger a wave-wide refill.  On 2^22 rays through 2^20
+// triangles (closest hit) 32 idle lanes cost 2%, 48 gain 1% and cost 1% on the
+// cornell frame; any hit over a million rays: 32 3% faster than 40, 48 4% slower.
+constexpr int kRefill = 40;
+constexpr int kRefillAny = 32;
+// A record step runs once this share of the walking lanes waits for one
+// (1 / n), else a node step.  Closest hit: a third (half: 4% slower, a
+// quarter: 0.5%); any hit, whose rays end at their first hit: half (a third:
+// 7% slower).
+constexpr int kVote = 3;
+constexpr int kVoteAny = 2;
 
 struct TraceArgs {
-    SceneView sv;
+    SceneView sv;  // first (cold_args)
     const float* o;
     const float* d;
     uint32_t n;
@@ -43,6 +50,11 @@ struct TraceArgs {
     float tmax;             // any-hit: hits at t >= tmax do not count
     int spill_cap;          // global spill entries per lane; a deeper stack hands the ray to the exact engine
 };
+
+// The kernel's arguments, for code outside the traversal loop (cold_scene).
+__device__ __forceinline__ const TraceArgs& cold_args(const TraceArgs& a) {
+    return *(const TraceArgs*)&cold_scene(a.sv);
+}
 
 __device__ __forceinline__ void write_out(const TraceArgs& a, uint32_t i, const HitOut& h) {
     if (a.prim) a.prim[i] = h.prim;
@@ -67,178 +79,182 @@ enum : int {
     kCtrFetch = 64,         // first ray-fetch partition counter
     kCtrWords = 1024,
 };
-// Dynamic ray fetch draws from kFetchParts partitions of the ray range, each
-// with its own counter on its own 128-byte line: with ~20 traversal steps per
-// ray, thousands of waves refilling through one counter serialise on that
-// address.  A wave starts on partition blockIdx % kFetchParts and moves on
-// when it runs dry.  Workgroups are dealt round-robin to the 8 XCDs, so a
-// partition's first waves all run on one XCD (blockIdx % 8) and adjacent rays
-// share that XCD's L2: 32 partitions (four per XCD) cost the coherent rays 13%.
-constexpr int kFetchParts = 16;  // 8 and 32 measured: equal and 4% slower
+// Ray fetch.  The rays are cut into blocks of 2^lb, dealt to kFetchParts parts
+// in turn; each part has its own waves (blockIdx mod kFetchParts) and its own
+// counter on its own 128-byte line.  Thousands of waves refilling through one
+// counter serialise on that address (about 20 ns an atomic), so no wave ever
+// draws from another part: dealing small blocks balances the parts instead (a
+// part holds some of every stretch of the launch's rays).  Parts cut as
+// stretches of the launch, with the waves of a finished part drawing from the
+// others, were 22% slower on the 512 x 512 cornell frame and 20% on a million
+// any-hit rays: at the end all waves meet on the counters that are left.
+// Workgroups are dealt round-robin to the 8 XCDs, so a part's waves all run on
+// one XCD and adjacent rays share its L2.
+constexpr uint32_t kLogFetchParts = 4;
+constexpr int kFetchParts = 1 << kLogFetchParts;
+constexpr uint32_t kLogFetchChunks = 4;    // a counter hands out 1/16 of a wave's share at a time ...
+constexpr uint32_t kMaxFetchChunk = 256;   // ... between 64 and 256 rays (64: the 2^27-path frame 1-6% slower)
+// Blocks of 2^lb <= 4,096 rays, at least 32 of them a part (2 or 4 a part: 2-3% slower).
+VR_HD uint32_t fetch_log_block(uint32_t n, uint32_t lparts) {
+    const uint32_t lg = 31u - (uint32_t)__builtin_clz(n | 1u);
+    const uint32_t lb = lg > lparts + 5u ? lg - lparts - 5u : 0u;
+    return lb > 12u ? 12u : lb;
+}
+// Items of part `part` of n.
+VR_HD uint32_t fetch_part_size(uint32_t n, uint32_t part, uint32_t lparts, uint32_t lb) {
+    const uint32_t round = lb + lparts, rest = n & ((1u << round) - 1u), at = part << lb;
+    const uint32_t tail = rest > at ? rest - at : 0u;
+    return ((n >> round) << lb) + (tail < (1u << lb) ? tail : 1u << lb);
+}
+// Item k of part `part`.
+VR_HD uint32_t fetch_item(uint32_t k, uint32_t part, uint32_t lparts, uint32_t lb) {
+    return ((((k >> lb) << lparts) | part) << lb) | (k & ((1u << lb) - 1u));
+}
 constexpr int kFetchStride = 32;  // words between two partition counters
 static_assert(kCtrFetch + kFetchParts * kFetchStride <= kCtrWords, "counter block too small");
 static_assert(kFetchParts <= 64, "one lane clears each partition counter");
 
 // Persistent wide-engine kernel: every lane runs its own ray as a resumable
-// state machine; each iteration is a node phase (up to kNodeSteps inner nodes)
-// followed by a leaf phase (one leaf's triangles); whenever kRefill lanes of
-// the wave are idle the wave fetches that many new rays with one atomic
-// (dynamic ray fetch), so long incoherent rays do not leave the wave idle.
-// A refill costs an atomic round trip plus the new rays' loads, and with a
-// spatial-split BVH a ray needs only ~20 steps, so refills wait until a
-// good part of the wave is idle (40 of 64 lanes, for closest and any hit)
-// and draw from partitioned counters (below).
+// state machine whose next step is a node or a triangle record.  In each
+// iteration the wave votes: a record step runs if enough of the walking lanes
+// wait for one (kVote), else a node step, so a good part of them takes part
+// in every step, whatever their rays need.  A ray that has ended waits in its lane until kRefill lanes of
+// the wave are idle; then all of them confirm and write their hits together
+// and the wave fetches as many new rays with one atomic (dynamic ray fetch).
 template <bool ANY, bool WT, bool INST>
 __device__ __forceinline__ void trace_persist(const TraceArgs& a) {
     constexpr int LDS = ANY ? kLdsStackAny : kLdsStack;
     __shared__ u32x2 lds[LDS * kWave];
     const int lane = threadIdx.x;
     const uint32_t glane = blockIdx.x * kWave + lane;
-    const WideStack ws{lds + lane, kWave, a.spill + glane, (int)a.spill_lanes, a.spill_cap};
-    const uint32_t kNone = 0xFFFFFFFFu;
+    const WideStack ws{(lds_u32x2*)(lds + lane), kWave, a.spill + glane, (int)a.spill_lanes, a.spill_cap};
     const uint32_t n = a.count ? *a.count : a.n;
     WideState st;
-    uint32_t ray = kNone;
-    bool exhausted = false;
-    uint32_t part = blockIdx.x % kFetchParts;  // wave-uniform
-    int dry = 0;                               // partitions found empty so far
+    uint32_t ray = 0;
+    // The lane's state as one word.  (As bools they were lane masks in
+    // scalar registers, which spilled: 3% slower.)
+    enum : uint32_t { kWalk = 0, kDone = 1, kExact = 2, kIdle = 3 };
+    uint32_t status = kIdle;
+    st.tg_mask = 0;
+    // Waves and blocks of 2^lb rays are dealt to the parts in turn.  A wave's
+    // first rays are its own by position, as many as an equal share of a small
+    // launch allows (at most 64): few rays are spread over all waves, where
+    // they end soonest, and nothing is fetched for them.  What the first rays
+    // of a part's waves leave of it is drawn from its counter in chunks.  (1 or
+    // kFetchParts parts and shifts: nothing divides but once.)
+    const uint32_t lparts = gridDim.x >= (uint32_t)kFetchParts ? kLogFetchParts : 0u, parts = 1u << lparts;
+    const uint32_t part = blockIdx.x & (parts - 1u);
+    const uint32_t waves = (gridDim.x - part + parts - 1u) >> lparts;  // of this part
+    const uint32_t lb = fetch_log_block(n, lparts);
+    const uint32_t size = fetch_part_size(n, part, lparts, lb);
+    const uint32_t share = size ? (size - 1u) / waves + 1u : 0u;
+    const uint32_t first = min(share, 64u), chunk = min(max(share >> kLogFetchChunks, 64u), kMaxFetchChunk);
+    // the wave's rays at hand: the part's [base, end)
+    uint32_t base = min(first * (blockIdx.x >> lparts), size), end = min(base + first, size);
+    bool dry = first * waves >= size, exhausted = false;  // nothing left to draw; and no ray at hand
     for (;;) {
-        bool idle = ray == kNone;
-        uint64_t idle_mask = __ballot(idle);
-        int nidle = __popcll(idle_mask);
-        if (!exhausted && nidle >= (ANY ? kRefillAny : kRefill)) {
-            // take nidle rays from the current partition, moving on while it is empty
-            uint32_t base = 0, hi = 0;
-            for (;;) {
-                const uint32_t lo = (uint32_t)((uint64_t)n * part / kFetchParts);
-                hi = (uint32_t)((uint64_t)n * (part + 1) / kFetchParts);
+        const uint64_t walking = __ballot(status == kWalk);
+        if (walking == 0ull || (!exhausted && 64 - __popcll(walking) >= (ANY ? kRefillAny : kRefill))) {
+            const TraceArgs& c = cold_args(a);
+            // finished rays: confirm and write, or hand over to the exact engine
+            if (status == kDone || status == kExact) {
+                HitOut h;
+                int rc = status == kExact ? kStepFallback : wide_finish<ANY, WT, INST>(c.sv, st, c.tmin, h);
+                if (rc == kStepFallback) {
+                    uint32_t slot = atomicAdd(c.fb_count, 1u);
+                    c.fb_list[slot] = ray;
+                } else {
+                    write_out(c, ray, h);
+                }
+                status = kIdle;
+            }
+            if (exhausted) break;  // (no lane walks)
+            const uint64_t idle_mask = ~walking;
+            const uint32_t nidle = (uint32_t)__popcll(idle_mask);
+            // rays at hand, and if they do not suffice a new chunk [nbase, nend)
+            const uint32_t avail = end - base;
+            uint32_t nbase = 0, nend = 0;
+            if (avail < nidle && !dry) {
                 uint32_t got = 0;
-                if (lane == 0) got = atomicAdd(a.next + part * kFetchStride, (uint32_t)nidle);
-                base = lo + __shfl(got, 0);
-                if (base < hi) break;
-                if (++dry == kFetchParts) {
-                    exhausted = true;
-                    break;
-                }
-                part = part + 1 == (uint32_t)kFetchParts ? 0u : part + 1;
+                if (lane == 0) got = atomicAdd(c.next + part * kFetchStride, chunk);
+                nbase = min(first * waves + __shfl(got, 0), size);
+                nend = min(nbase + chunk, size);
+                dry = nend == size;
             }
-            if (idle && !exhausted) {
-                uint32_t k = base + (uint32_t)__popcll(idle_mask & ((1ull << lane) - 1ull));
-                if (k < hi) {
-                    uint32_t r = a.queue ? a.queue[k] : k;
-                    ray = r;
-                    vf3 o = mk3(a.o[3 * r], a.o[3 * r + 1], a.o[3 * r + 2]);
-                    vf3 d = mk3(a.d[3 * r], a.d[3 * r + 1], a.d[3 * r + 2]);
-                    wide_init<WT>(st, o, d, a.sv.num_qnodes > 0);
-                    if (a.sv.num_analytic) wide_seed_analytic<ANY, WT>(a.sv, st, a.tmin, a.tmax);
-                }
+            const uint32_t rank = (uint32_t)__popcll(idle_mask & ((1ull << lane) - 1ull));
+            const uint32_t k = rank < avail ? base + rank : nbase + (rank - avail);
+            if (status == kIdle && (rank < avail || k < nend)) {
+                const uint32_t item = fetch_item(k, part, lparts, lb);
+                ray = c.queue ? c.queue[item] : item;
+                status = kWalk;
+                vf3 o = mk3(c.o[3 * ray], c.o[3 * ray + 1], c.o[3 * ray + 2]);
+                vf3 d = mk3(c.d[3 * ray], c.d[3 * ray + 1], c.d[3 * ray + 2]);
+                wide_init<WT>(st, o, d, c.sv.num_qnodes > 0);
+                if (c.sv.num_analytic) wide_seed_analytic<ANY, WT>(c.sv, st, c.tmin, c.tmax);
             }
-        }
-        if (exhausted && __ballot(ray != kNone) == 0ull) break;
-        // Node phase (while-while traversal with leaf postponement, Aila &
-        // Laine 2009): lanes walk inner nodes together; a lane that reaches a
-        // leaf parks it and keeps walking until it meets a second leaf; the
-        // phase ends once no lane is still looking for its first leaf.  Node
-        // and triangle work then run in separate passes instead of splitting
-        // every iteration between the two.
-        // The lane's state as one word: 0 walking, 1 done, 2 handed to the
-        // exact engine, 3 no ray.  (As three bools they were three lane
-        // masks in scalar registers, which spilled: 3% slower.)
-        uint32_t status = ray != kNone ? 0u : 3u;
-        uint32_t leaf = kNone;
-        for (int it = 0; it < kNodeSteps; ++it) {
-            const bool searching = status == 0u && leaf == kNone;
-            if (__ballot(searching) == 0ull) break;
-            if (status != 0u) continue;
-            if (!st.have) {
-                if (!wide_pop_next<LDS, ANY>(st, ws)) {
-                    if (leaf == kNone) status = 1u;  // stack empty, nothing parked: the ray is finished
-                    continue;
-                }
-            }
-            if (st.cur & kLeafBit) {
-                if (leaf == kNone) {  // park the first leaf, keep walking
-                    leaf = st.cur;
-                    st.have = false;
-                }
-                continue;  // a second leaf waits in st.cur
-            }
-            if (INST && (st.cur & kInstEntry)) {
-                // entering or leaving an instance changes the ray: a parked
-                // leaf is tested with the current one first (the entry waits)
-                if (leaf != kNone) continue;
-                st.have = false;
-                if (st.cur == kInstExit) {  // back to the world ray, reloaded
-                    wide_instance_exit<WT>(st, mk3(a.o[3 * ray], a.o[3 * ray + 1], a.o[3 * ray + 2]),
-                                           mk3(a.d[3 * ray], a.d[3 * ray + 1], a.d[3 * ray + 2]));
-                } else if (wide_instance_enter<LDS, WT>(a.sv, st, ws, st.cur, a.tmin) == kStepFallback) {
-                    status = 2u;
-                }
-                continue;
-            }
-            st.have = false;
-            if (wide_node<LDS, ANY>(a.sv, st, ws, st.cur, a.tmin, a.tmax) == kStepFallback) status = 2u;
-        }
-        // Leaf phase
-        if (leaf != kNone && status != 2u) {
-            const int rc = wide_leaf<LDS, ANY, WT, INST>(a.sv, st, ws, leaf, a.tmin, a.tmax);
-            if (rc == kStepDone) status = 1u;
-            else if (rc == kStepFallback) status = 2u;
-        }
-        if (status == 0u && !st.have && st.sp == 0) status = 1u;
-        if (status == 1u || status == 2u) {
-            HitOut h;
-            int rc = status == 2u ? kStepFallback : wide_finish<ANY, WT, INST>(a.sv, st, a.tmin, h);
-            if (rc == kStepFallback) {
-                uint32_t slot = atomicAdd(a.fb_count, 1u);
-                a.fb_list[slot] = ray;
+            if (avail < nidle) {
+                base = min(nbase + (nidle - avail), nend);
+                end = nend;
             } else {
-                write_out(a, ray, h);
+                base += nidle;
             }
-            ray = kNone;
+            exhausted = dry && base == end;
+            continue;
+        }
+        const uint64_t tri = __ballot(status == kWalk && st.tg_mask != 0u);
+        if ((ANY ? kVoteAny : kVote) * __popcll(tri) >= __popcll(walking)) {
+            if (status == kWalk && st.tg_mask != 0u)
+                status = (uint32_t)wide_tri_step<LDS, ANY, WT, INST>(a.sv, st, ws, a.tmin, a.tmax);
+        } else {
+            if (status == kWalk && st.tg_mask == 0u)
+                status = (uint32_t)wide_node_step<LDS, ANY, WT, INST>(a.sv, st, ws, a.tmin, a.tmax, [&](vf3& wo, vf3& wd) {
+                    const TraceArgs& c = cold_args(a);
+                    wo = mk3(c.o[3 * ray], c.o[3 * ray + 1], c.o[3 * ray + 2]);
+                    wd = mk3(c.d[3 * ray], c.d[3 * ray + 1], c.d[3 * ray + 2]);
+                });
         }
     }
 }
 
-// Closest hit: registers held to what 8 waves per SIMD allow (64 VGPRs, no
-// scratch; the 5 KB LDS ring allows 8 as well).  Any hit keeps the registers
-// it wants (72 VGPRs, 7 waves; its 6 KB ring allows 6.7 per SIMD): held to 64
-// it spills.
+// Registers held to 7 waves per SIMD (72 VGPRs, no scratch).  The kernel waits
+// for memory as much as it issues: at 3, 4, 5 and 6 waves the 2^27-path terrain
+// frame took 30%, 16%, 8% and 1% longer; at 8 waves it spills.
 template <bool ANY, bool WT = false, bool INST = false>
 __global__ void k_trace_persist(TraceArgs a);
 template <>
-__global__ __launch_bounds__(kWave, 8) void k_trace_persist<false, false, false>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 7) void k_trace_persist<false, false, false>(TraceArgs a) {
     trace_persist<false, false, false>(a);
 }
 template <>
-__global__ __launch_bounds__(kWave) void k_trace_persist<true, false, false>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 7) void k_trace_persist<true, false, false>(TraceArgs a) {
     trace_persist<true, false, false>(a);
 }
 // watertight engine (extended estimator only)
 template <>
-__global__ __launch_bounds__(kWave, 8) void k_trace_persist<false, true, false>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 7) void k_trace_persist<false, true, false>(TraceArgs a) {
     trace_persist<false, true, false>(a);
 }
 template <>
-__global__ __launch_bounds__(kWave) void k_trace_persist<true, true, false>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 7) void k_trace_persist<true, true, false>(TraceArgs a) {
     trace_persist<true, true, false>(a);
 }
-// scenes with instances (the instance bookkeeping needs a few more
-// registers: held to 8 waves per SIMD the closest-hit kernels spill)
+// scenes with instances (the instance bookkeeping needs more registers, about
+// 110: held to 5 to 7 waves per SIMD the kernels spill, and a 960 x 540 x 4
+// frame of 200 instances took 11.1 ms instead of 6.9)
 template <>
-__global__ __launch_bounds__(kWave, 7) void k_trace_persist<false, false, true>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 4) void k_trace_persist<false, false, true>(TraceArgs a) {
     trace_persist<false, false, true>(a);
 }
 template <>
-__global__ __launch_bounds__(kWave, 6) void k_trace_persist<true, false, true>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 4) void k_trace_persist<true, false, true>(TraceArgs a) {
     trace_persist<true, false, true>(a);
 }
 template <>
-__global__ __launch_bounds__(kWave, 6) void k_trace_persist<false, true, true>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 4) void k_trace_persist<false, true, true>(TraceArgs a) {
     trace_persist<false, true, true>(a);
 }
 template <>
-__global__ __launch_bounds__(kWave) void k_trace_persist<true, true, true>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 4) void k_trace_persist<true, true, true>(TraceArgs a) {
     trace_persist<true, true, true>(a);
 }
 
@@ -546,7 +562,7 @@ static int launch_trace_with(vr_scene* s, const TraceJob& j, const TraceScratch&
         int rc = persist_grid(s, j.any, wt, blocks);
         if (rc) return rc;
         blocks = std::min<uint32_t>(blocks, sc.spill_lanes / kWave);
-        blocks = std::min<uint32_t>(blocks, (j.n_max + kWave - 1) / kWave);
+        blocks = std::min<uint32_t>(blocks, j.n_max);
         void (*persist)(TraceArgs) =
             kPersistKernels[(j.any ? 1 : 0) + (wt ? 2 : 0) + (s->view.num_instances > 0 ? 4 : 0)];
         void (*exact)(TraceArgs, const uint32_t*, uint32_t*, uint32_t*, uint64_t*) =

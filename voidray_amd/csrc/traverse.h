@@ -3,7 +3,7 @@
 //
 // Two engines answer SceneAcceleration::hit (core/scene.rs:182-185):
 //
-//  * wide  — SAH 4-wide BVH with 8-bit outward-rounded child boxes, one ray
+//  * wide  — SAH 8-wide BVH with 8-bit outward-rounded child boxes, one ray
 //            per lane, a short LDS stack, nearest-child-first order and t_max
 //            shrinking.  Box tests are conservative (padded boxes, a relative
 //            slack on the slab exit, a relative slack on the cull distance), so
@@ -32,7 +32,7 @@
 //
 // Instances (template flag INST, scenes with vr_instance surfaces; no
 // counterpart in the reference): an instance is one record of the top-level
-// wide BVH holding its world box (kInstanceMarker in p2.x).  A leaf that meets
+// wide BVH holding its world box (kInstanceMarker in p2.x).  A ray that meets
 // one pushes an "enter" entry at the box's entry distance; popping it pushes an
 // "exit" entry, maps the ray into the instance's object space (t is unchanged:
 // the direction is mapped, not renormalised) and walks the shared object-space
@@ -54,6 +54,21 @@ struct HitOut {
     float t, u, v;
     uint32_t prim;  // 0xFFFFFFFF: miss
 };
+
+// The scene, for code that rarely runs in a kernel whose first argument starts
+// with a SceneView (TraceArgs): read through a pointer the compiler cannot see
+// through, so that it loads what the code needs there and then.  Through the
+// argument itself it keeps all of it in scalar registers across the traversal
+// loop, spills them and reads them back, lane by lane, in every step.
+VR_HD const SceneView& cold_scene(const SceneView& sv) {
+#ifdef __HIP_DEVICE_COMPILE__
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const SceneView*)p;
+#else
+    return sv;
+#endif
+}
 
 constexpr float kSlabSlack = 1.0f + 1.0f / 131072.0f;  // 2^-17 relative on the slab exit
 constexpr float kCullSlack = 1.0f + 1.0f / 65536.0f;   // 2^-16 relative on t_best
@@ -203,24 +218,30 @@ VR_HD int analytic_best(const SceneView& sv, vf3 o, vf3 d, float tmin, float fir
 constexpr uint32_t kAnalyticSlot = 0x40000000u;  // best_slot of an analytic winner (triangle slots < 2^27)
 
 // ---- wide engine as a resumable per-lane state machine ----------------------
-// The stack lives in LDS (LDS_STACK entries per lane, strided by `stride`) and
-// spills its oldest entries to a per-lane global region (`spill`, strided by
-// `spill_stride`, `spill_cap` entries) when it overflows.  Each entry is
-// (node or leaf code, bits of the entry distance) so a popped subtree that
-// lies beyond the current best hit is skipped without touching its node.
+// A ray holds the node it visits next and a triangle group (the records of
+// the hit leaves of one wide node); a step visits a node (wide_node_step) or
+// tests one record (wide_tri_step).  A node's nearest hit inner child is
+// visited next; the others go on the stack together as one 8-byte entry: the
+// node's first child, the mask of the hit children and a lower bound of their
+// entry distances, so a pop skips the group when all of it lies beyond the
+// best hit.  One entry per level at most.  The stack's first LDS_STACK entries
+// live in LDS (strided by `stride`), deeper ones in a per-lane global region
+// (`spill`, strided by `spill_stride`, `spill_cap` entries).
 struct WideState {
     vf3 o, d;  // the ray as the current BVH sees it (object space inside an instance)
     WTRay wt;  // watertight mode: the ray's shear (unused otherwise)
     float idx, idy, idz;
     float tbest, bu, bv;
     uint32_t best_prim, best_slot;
-    uint32_t cur;
-    int sp, lo;
-    int top;  // LDS ring slot of entry sp (sp modulo the ring size, kept incrementally)
+    uint32_t cur;  // node to visit next, kNoNode: the stack decides
+    // triangle group: first record, the positions (QNode::leaf_bits) of the
+    // records to test and of the node's records
+    uint32_t tg_base, tg_mask, tg_all;
+    int sp;
     // 0 or 1.  As words they live in vector registers; as bools the compiler
     // keeps each as a lane mask in scalar registers, which the persistent
     // kernel runs out of (spilled masks cost readlanes in every node step).
-    uint32_t have, unconfirmed, found;
+    uint32_t unconfirmed, found;
     // INST only: the instance being walked (kNoInstance: none), its prim
     // base and triangle determinant threshold, the instance of the best hit
     // (the world ray is the caller's)
@@ -228,13 +249,26 @@ struct WideState {
     float inst_eps;
 };
 constexpr uint32_t kNoInstance = 0xFFFFFFFFu;
-// Stack codes of instance entries (INST): bit 30 set, below the leaf bit.
-// Node indices stay below 2^30 (the scene build checks it).
+// First words of instance stack entries (INST): bit 30 set.  Node indices
+// stay below 2^29 (the scene build checks it).
 constexpr uint32_t kInstEntry = 0x40000000u;            // | instance index: enter
 constexpr uint32_t kInstExit = kInstEntry | 0x3FFFFFFFu;  // leave the current instance
+// Group entries: x = first child | kDescend, y = bits 16..31 of the bound's
+// float bits (rounded down) | hit children by slot.
+constexpr uint32_t kDescend = 0x80000000u;  // the far slots come first (the ray runs against the node's axis)
+constexpr uint32_t kNoNode = 0xFFFFFFFFu;
 
+// On the device the stack's LDS part is addressed through an LDS pointer: with
+// a generic one the compiler merges the two stores of a push (and the two
+// loads of a pop) into one flat access through a selected pointer, which
+// takes the slower path and waits for both memories.
+#ifdef __HIP_DEVICE_COMPILE__
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+#else
+typedef u32x2 lds_u32x2;
+#endif
 struct WideStack {
-    u32x2* lds;
+    lds_u32x2* lds;
     int stride;
     u32x2* spill;
     int spill_stride, spill_cap;
@@ -263,11 +297,11 @@ VR_HD void wide_init(WideState& st, vf3 o, vf3 d, bool nonempty) {
     st.bu = st.bv = 0.f;
     st.best_prim = 0xFFFFFFFFu;
     st.best_slot = 0xFFFFFFFFu;
-    st.cur = 0;
+    st.cur = nonempty ? 0u : kNoNode;
+    st.tg_base = 0;
+    st.tg_mask = 0;
+    st.tg_all = 0;
     st.sp = 0;
-    st.lo = 0;
-    st.top = 0;
-    st.have = nonempty;
     st.unconfirmed = false;
     st.found = false;
 }
@@ -285,7 +319,7 @@ VR_HD void wide_seed_analytic(const SceneView& sv, WideState& st, float tmin, fl
     if (ANY) {
         if (!(t < tmax_any)) return;
         st.found = true;
-        st.have = false;
+        st.cur = kNoNode;
     }
     st.tbest = t;
     st.best_prim = prim;
@@ -294,111 +328,89 @@ VR_HD void wide_seed_analytic(const SceneView& sv, WideState& st, float tmin, fl
     st.bv = v;
 }
 
-// The LDS part of the stack is a ring of LDS_STACK entries: entry i lives in
-// slot i mod LDS_STACK, and st.top tracks the slot of entry st.sp without a
-// division.  When the ring is full (sp - lo == LDS_STACK) the slot of entry sp
-// is that of the oldest LDS entry lo, which moves to the spill region first.
 template <int LDS_STACK>
 VR_HD bool wide_push(WideState& st, const WideStack& ws, u32x2 e) {
-    if (st.sp - st.lo == LDS_STACK) {
-        if (st.lo >= ws.spill_cap) return false;
-        ws.spill[st.lo * ws.spill_stride] = ws.lds[st.top * ws.stride];
-        ++st.lo;
+    if (st.sp < LDS_STACK) {
+        ws.lds[st.sp * ws.stride] = e;
+    } else {
+        if (st.sp - LDS_STACK >= ws.spill_cap) return false;
+        ws.spill[(st.sp - LDS_STACK) * ws.spill_stride] = e;
     }
-    ws.lds[st.top * ws.stride] = e;
     ++st.sp;
-    st.top = st.top + 1 == LDS_STACK ? 0 : st.top + 1;
     return true;
 }
 
+// The stack's top entry (sp > 0), which stays there.
 template <int LDS_STACK>
-VR_HD u32x2 wide_pop(WideState& st, const WideStack& ws) {
-    --st.sp;
-    st.top = st.top == 0 ? LDS_STACK - 1 : st.top - 1;
-    if (st.sp < st.lo) {
-        st.lo = st.sp;
-        return ws.spill[st.sp * ws.spill_stride];
-    }
-    return ws.lds[st.top * ws.stride];
+VR_HD u32x2 wide_top(const WideState& st, const WideStack& ws) {
+    const int i = st.sp - 1;
+    if (i >= LDS_STACK) return ws.spill[(i - LDS_STACK) * ws.spill_stride];
+    return ws.lds[i * ws.stride];
+}
+template <int LDS_STACK>
+VR_HD void wide_set_top(const WideState& st, const WideStack& ws, u32x2 e) {
+    const int i = st.sp - 1;
+    if (i >= LDS_STACK) ws.spill[(i - LDS_STACK) * ws.spill_stride] = e;
+    else ws.lds[i * ws.stride] = e;
 }
 
-// Pops the nearest pending entry that survives culling into st.cur; false
-// when the stack is empty.
-template <int LDS_STACK, bool ANY>
-VR_HD bool wide_pop_next(WideState& st, const WideStack& ws) {
-    while (st.sp > 0) {
-        u32x2 e = wide_pop<LDS_STACK>(st, ws);
-        if (!ANY && u2f(e.y) > st.tbest * kCullSlack) continue;
-        st.cur = e.x;
-        st.have = true;
-        return true;
-    }
-    return false;
-}
-
-// Tests the triangles of leaf `code`.  Returns kStepContinue, kStepDone when
-// an any-hit query has its confirmed hit, or kStepFallback when an instance
-// entry finds the stack exhausted (INST).
+// Tests one record of the triangle group (tg_mask != 0).  Returns
+// kStepContinue, kStepDone when an any-hit query has its confirmed hit, or
+// kStepFallback when an instance entry finds the stack exhausted (INST).
 template <int LDS_STACK, bool ANY, bool WT = false, bool INST = false>
-VR_HD int wide_leaf(const SceneView& sv, WideState& st, const WideStack& ws, uint32_t code, float tmin,
-                    float tmax_any) {
+VR_HD int wide_tri_step(const SceneView& sv, WideState& st, const WideStack& ws, float tmin, float tmax_any) {
     const vf3 o = st.o, d = st.d;
     const bool in_inst = INST && st.inst != kNoInstance;
-    uint32_t first = code & 0x07FFFFFFu;
-    uint32_t cnt = ((code >> 27) & 7u) + 1u;
-    for (uint32_t k = 0; k < cnt; ++k) {
-        // the record's index (best_slot keeps it, not the leaf entry)
-        const uint32_t slot = sv.tri_ref ? sv.tri_ref[first + k] : first + k;
-        vf3 p0, p1, p2;
-        load_tri_geom(sv.tris, slot, p0, p1, p2);
-        if (INST && f2u(p2.x) == kInstanceMarker) {
-            // an instance: its world box is [p0, p1]; enter it later, in
-            // near-to-far order with the other pending entries
-            const float tcull = ANY ? tmax_any : st.tbest * kCullSlack;
-            const float ax = (p0.x - o.x) * st.idx, bx = (p1.x - o.x) * st.idx;
-            const float ay = (p0.y - o.y) * st.idy, by = (p1.y - o.y) * st.idy;
-            const float az = (p0.z - o.z) * st.idz, bz = (p1.z - o.z) * st.idz;
-            const float tnear = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fmaxf(fminf(az, bz), tmin));
-            const float tfar = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fminf(fmaxf(az, bz), tcull));
-            if (tnear <= tfar * kSlabSlack &&
-                !wide_push<LDS_STACK>(st, ws, u32x2{kInstEntry | f2u(p2.y), f2u(tnear)}))
-                return kStepFallback;
-            continue;
-        }
-        MTResult r;
-        if (WT ? !wt_hit(st.wt, o, p0, p1, p2, tmin, r)
-               : !mt_hit(o, d, p0, p1, p2, tmin, r, in_inst ? st.inst_eps : -1.0f))
-            continue;
-        if (ANY) {
-            if (r.t < tmax_any) {
-                if (WT || in_inst ||
-                    confirm_winner(sv, o, d, tmin, r.t, p0, p1, p2, tri_word(sv.tris, slot, 11),
-                                   tri_word(sv.tris, slot, 9))) {
-                    st.found = true;
-                    st.tbest = r.t;
-                    st.best_slot = slot;
-                    st.bu = r.u;
-                    st.bv = r.v;
-                    if (INST) {
-                        st.best_inst = st.inst;
-                        st.best_prim = st.inst_base + tri_word(sv.tris, slot, 9);
-                    }
-                    return kStepDone;
-                }
-                st.unconfirmed = true;
-            }
-            continue;
-        }
-        if (r.t > st.tbest) continue;
-        const uint32_t prim = (in_inst ? st.inst_base : 0u) + tri_word(sv.tris, slot, 9);
-        if (r.t < st.tbest || prim < st.best_prim) {
+    const uint32_t bit = st.tg_mask & (0u - st.tg_mask);
+    const uint32_t entry = st.tg_base + (uint32_t)__builtin_popcount(st.tg_all & (bit - 1u));
+    st.tg_mask ^= bit;
+    // the record's index (best_slot keeps it, not the leaf entry)
+    const uint32_t slot = sv.tri_ref ? sv.tri_ref[entry] : entry;
+    vf3 p0, p1, p2;
+    load_tri_geom(sv.tris, slot, p0, p1, p2);
+    if (INST && f2u(p2.x) == kInstanceMarker) {
+        // an instance: its world box is [p0, p1]; entered when its stack entry is popped
+        const float tcull = ANY ? tmax_any : st.tbest * kCullSlack;
+        const float ax = (p0.x - o.x) * st.idx, bx = (p1.x - o.x) * st.idx;
+        const float ay = (p0.y - o.y) * st.idy, by = (p1.y - o.y) * st.idy;
+        const float az = (p0.z - o.z) * st.idz, bz = (p1.z - o.z) * st.idz;
+        const float tnear = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fmaxf(fminf(az, bz), tmin));
+        const float tfar = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fminf(fmaxf(az, bz), tcull));
+        if (tnear <= tfar * kSlabSlack && !wide_push<LDS_STACK>(st, ws, u32x2{kInstEntry | f2u(p2.y), f2u(tnear)}))
+            return kStepFallback;
+        return kStepContinue;
+    }
+    MTResult r;
+    if (WT ? !wt_hit(st.wt, o, p0, p1, p2, tmin, r) : !mt_hit(o, d, p0, p1, p2, tmin, r, in_inst ? st.inst_eps : -1.0f))
+        return kStepContinue;
+    if (ANY) {
+        if (!(r.t < tmax_any)) return kStepContinue;
+        if (WT || in_inst ||
+            confirm_winner(cold_scene(sv), o, d, tmin, r.t, p0, p1, p2, tri_word(sv.tris, slot, 11),
+                           tri_word(sv.tris, slot, 9))) {
+            st.found = true;
             st.tbest = r.t;
-            st.best_prim = prim;
             st.best_slot = slot;
             st.bu = r.u;
             st.bv = r.v;
-            if (INST) st.best_inst = st.inst;
+            if (INST) {
+                st.best_inst = st.inst;
+                st.best_prim = st.inst_base + tri_word(sv.tris, slot, 9);
+            }
+            return kStepDone;
         }
+        st.unconfirmed = true;
+        return kStepContinue;
+    }
+    if (r.t > st.tbest) return kStepContinue;
+    const uint32_t prim = (in_inst ? st.inst_base : 0u) + tri_word(sv.tris, slot, 9);
+    if (r.t < st.tbest || prim < st.best_prim) {
+        st.tbest = r.t;
+        st.best_prim = prim;
+        st.best_slot = slot;
+        st.bu = r.u;
+        st.bv = r.v;
+        if (INST) st.best_inst = st.inst;
     }
     return kStepContinue;
 }
@@ -412,7 +424,7 @@ template <int LDS_STACK, bool WT = false>
 VR_HD int wide_instance_enter(const SceneView& sv, WideState& st, const WideStack& ws, uint32_t code, float tmin) {
     const uint32_t k = code & ~kInstEntry;
     if (!wide_push<LDS_STACK>(st, ws, u32x2{kInstExit, 0u})) return kStepFallback;
-    const InstanceDev& x = sv.instances[k];
+    const InstanceDev& x = cold_scene(sv).instances[k];
     vf3 oo, dd;
     instance_ray(x, st.o, st.d, oo, dd);
     wide_set_ray<WT>(st, oo, dd);
@@ -420,7 +432,6 @@ VR_HD int wide_instance_enter(const SceneView& sv, WideState& st, const WideStac
     st.inst_base = x.prim_base;
     st.inst_eps = tmin * x.det_inv;
     st.cur = x.blas_root;
-    st.have = true;
     return kStepContinue;
 }
 
@@ -430,88 +441,135 @@ VR_HD void wide_instance_exit(WideState& st, vf3 world_o, vf3 world_d) {
     st.inst = kNoInstance;
 }
 
-// Visits inner node `cur`: children in near-to-far order, the nearest becomes
-// st.cur (st.have), the others are pushed.  Returns kStepContinue, or
-// kStepFallback when the stack is exhausted (the exact engine answers).
-template <int LDS_STACK, bool ANY>
-VR_HD int wide_node(const SceneView& sv, WideState& st, const WideStack& ws, uint32_t cur, float tmin,
-                    float tmax_any) {
-    const vf3 o = st.o, d = st.d;
-    const u32x4* qp = (const u32x4*)(sv.qnodes + cur);
-    u32x4 w0 = qp[0], w1 = qp[1], w2 = qp[2], w3 = qp[3];
-    uint32_t e = w0.w;
-    float sx = u2f((e & 0xFFu) << 23) * st.idx;
-    float sy = u2f(((e >> 8) & 0xFFu) << 23) * st.idy;
-    float sz = u2f(((e >> 16) & 0xFFu) << 23) * st.idz;
-    float bx = (u2f(w0.x) - o.x) * st.idx;
-    float by = (u2f(w0.y) - o.y) * st.idy;
-    float bz = (u2f(w0.z) - o.z) * st.idz;
-    uint32_t ch[4] = {w1.x, w1.y, w1.z, w1.w};
-    // Near and far planes chosen once per node from the ray's direction signs
-    // (all four children's bytes at once): with s > 0, fma(lo, s, b) <=
-    // fma(hi, s, b), so this equals taking min/max per child and axis.
-    const bool negx = st.idx < 0.f, negy = st.idy < 0.f, negz = st.idz < 0.f;
-    uint32_t qnx = negx ? w2.w : w2.x, qfx = negx ? w2.x : w2.w;
-    uint32_t qny = negy ? w3.x : w2.y, qfy = negy ? w2.y : w3.x;
-    uint32_t qnz = negz ? w3.y : w2.z, qfz = negz ? w2.z : w3.y;
-    float tcull = ANY ? tmax_any : st.tbest * kCullSlack;
-    float tn[4];
-    uint32_t cid[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        float nx = fmaf((float)((qnx >> (8 * c)) & 0xFFu), sx, bx), fx = fmaf((float)((qfx >> (8 * c)) & 0xFFu), sx, bx);
-        float ny = fmaf((float)((qny >> (8 * c)) & 0xFFu), sy, by), fy = fmaf((float)((qfy >> (8 * c)) & 0xFFu), sy, by);
-        float nz = fmaf((float)((qnz >> (8 * c)) & 0xFFu), sz, bz), fz = fmaf((float)((qfz >> (8 * c)) & 0xFFu), sz, bz);
-        float tnear = fmaxf(fmaxf(nx, ny), fmaxf(nz, tmin));
-        float tfar = fminf(fminf(fx, fy), fminf(fz, tcull));
-        bool hit = ch[c] != kInvalidChild && tnear <= tfar * kSlabSlack;
-        tn[c] = hit ? tnear : kInf;
-        cid[c] = ch[c];
-    }
-    // sort (tnear, child) ascending; misses carry +inf and sink to the end
-#define VR_CSWAP(a, b)                                   \
-    if (tn[b] < tn[a]) {                                 \
-        float tt = tn[a];                                \
-        tn[a] = tn[b];                                   \
-        tn[b] = tt;                                      \
-        uint32_t cc = cid[a];                            \
-        cid[a] = cid[b];                                 \
-        cid[b] = cc;                                     \
-    }
-    VR_CSWAP(0, 1)
-    VR_CSWAP(2, 3)
-    VR_CSWAP(0, 2)
-    VR_CSWAP(1, 3)
-    VR_CSWAP(1, 2)
-#undef VR_CSWAP
-    if (tn[0] == kInf) return kStepContinue;
-    st.cur = cid[0];
-    st.have = true;
-    bool ok = true;
-#pragma unroll
-    for (int c = 3; c >= 1; --c) {
-        if (tn[c] == kInf) continue;
-        ok = ok && wide_push<LDS_STACK>(st, ws, u32x2{cid[c], f2u(tn[c])});
-    }
-    return ok ? kStepContinue : kStepFallback;
+VR_HD uint32_t min_u(uint32_t a, uint32_t b) { return a < b ? a : b; }
+// Median of three.
+VR_HD uint32_t med3_u(uint32_t a, uint32_t b, uint32_t c) {
+#ifdef __HIP_DEVICE_COMPILE__
+    uint32_t r;
+    asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    const uint32_t lo = a < b ? a : b, hi = a < b ? b : a;
+    return c < lo ? lo : c > hi ? hi : c;
+#endif
 }
 
-// One traversal step (one node or one leaf).  Returns kStepContinue,
-// kStepDone (result ready for wide_finish) or kStepFallback.
-// (wo, wd): the query's world ray, for leaving an instance (INST).
-template <int LDS_STACK, bool ANY, bool WT = false, bool INST = false>
-VR_HD int wide_step(const SceneView& sv, WideState& st, const WideStack& ws, float tmin, float tmax_any, vf3 wo,
-                    vf3 wd) {
-    if (!st.have && !wide_pop_next<LDS_STACK, ANY>(st, ws)) return kStepDone;
-    st.have = false;
-    const uint32_t cur = st.cur;
-    if (cur & kLeafBit) return wide_leaf<LDS_STACK, ANY, WT, INST>(sv, st, ws, cur, tmin, tmax_any);
-    if (INST && cur == kInstExit) {
-        wide_instance_exit<WT>(st, wo, wd);
-        return kStepContinue;
+// Tests the 8 child boxes of node `node`.  The hit leaves' records become the
+// triangle group, the nearest hit inner child (any hit: the first along the
+// node's axis) st.cur, and the other hit inner children are pushed.  Returns
+// kStepContinue, or kStepFallback when the stack is exhausted.
+template <int LDS_STACK, bool ANY>
+VR_HD int wide_node(const SceneView& sv, WideState& st, const WideStack& ws, uint32_t node, float tmin,
+                    float tmax_any) {
+    const u32x4* qp = (const u32x4*)(sv.qnodes + node);
+    const u32x4 w0 = qp[0], w1 = qp[1], w2 = qp[2], w3 = qp[3], w4 = qp[4];
+    const uint32_t e = w0.w;
+    const float sx = u2f((e & 0xFFu) << 23) * st.idx;
+    const float sy = u2f(((e >> 8) & 0xFFu) << 23) * st.idy;
+    const float sz = u2f(((e >> 16) & 0xFFu) << 23) * st.idz;
+    const uint32_t num_inner = e >> 24;
+    const float bx = (u2f(w0.x) - st.o.x) * st.idx;
+    const float by = (u2f(w0.y) - st.o.y) * st.idy;
+    const float bz = (u2f(w0.z) - st.o.z) * st.idz;
+    // Near and far planes chosen once per node from the ray's direction signs
+    // (four children's bytes at once): with s > 0, fma(lo, s, b) <=
+    // fma(hi, s, b), so this equals taking min/max per child and axis.
+    const bool negx = st.idx < 0.f, negy = st.idy < 0.f, negz = st.idz < 0.f;
+    const float tcull = ANY ? tmax_any : st.tbest * kCullSlack;
+    uint32_t hits = 0;
+    // the two smallest (entry distance, slot) keys of the hit inner children:
+    // the distance's float bits with the slot in the lowest three
+    uint32_t m1 = 0xFFFFFFFFu, m2 = 0xFFFFFFFFu;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        // words: lo x, y, z at 0..5, hi x, y, z at 6..11 of w2, w3, w4
+        const uint32_t lx = h ? w2.y : w2.x, ly = h ? w2.w : w2.z, lz = h ? w3.y : w3.x;
+        const uint32_t hx = h ? w3.w : w3.z, hy = h ? w4.y : w4.x, hz = h ? w4.w : w4.z;
+        const uint32_t qnx = negx ? hx : lx, qfx = negx ? lx : hx;
+        const uint32_t qny = negy ? hy : ly, qfy = negy ? ly : hy;
+        const uint32_t qnz = negz ? hz : lz, qfz = negz ? lz : hz;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int s = 4 * h + c;
+            const float nx = fmaf((float)((qnx >> (8 * c)) & 0xFFu), sx, bx), fx = fmaf((float)((qfx >> (8 * c)) & 0xFFu), sx, bx);
+            const float ny = fmaf((float)((qny >> (8 * c)) & 0xFFu), sy, by), fy = fmaf((float)((qfy >> (8 * c)) & 0xFFu), sy, by);
+            const float nz = fmaf((float)((qnz >> (8 * c)) & 0xFFu), sz, bz), fz = fmaf((float)((qfz >> (8 * c)) & 0xFFu), sz, bz);
+            const float tnear = fmaxf(fmaxf(nx, ny), fmaxf(nz, tmin));
+            const float tfar = fminf(fminf(fx, fy), fminf(fz, tcull));
+            const bool hit = tnear <= tfar * kSlabSlack;
+            hits |= hit ? 1u << s : 0u;
+            if (!ANY) {
+                const uint32_t key = hit && (uint32_t)s < num_inner ? (f2u(tnear) & ~7u) | (uint32_t)s : 0xFFFFFFFFu;
+                m2 = med3_u(m1, m2, key);
+                m1 = min_u(m1, key);
+            }
+        }
     }
-    if (INST && (cur & kInstEntry)) return wide_instance_enter<LDS_STACK, WT>(sv, st, ws, cur, tmin);
-    return wide_node<LDS_STACK, ANY>(sv, st, ws, cur, tmin, tmax_any);
+    // empty slots (lo 255, hi 0) can pass within the slack, or where a
+    // direction component is zero: only the node's own slots count
+    const uint32_t inner = (1u << num_inner) - 1u;
+    uint32_t leaves = hits & ~inner;
+    leaves = (leaves | (leaves << 8)) & 0x00F00Fu;
+    leaves = (leaves | (leaves << 4)) & 0x0C30C3u;
+    leaves = (leaves | (leaves << 2)) & 0x249249u;
+    st.tg_all = w1.z & 0xFFFFFFu;
+    st.tg_mask = ((leaves << 3) - leaves) & st.tg_all;
+    st.tg_base = w1.y;
+    hits &= inner;
+    st.cur = kNoNode;
+    if (hits) {
+        const uint32_t axis = (w1.z >> 24) & 3u;
+        const bool neg = axis == 0u ? negx : axis == 1u ? negy : negz;
+        uint32_t slot;
+        if (ANY) slot = neg ? 31u - (uint32_t)__builtin_clz(hits) : (uint32_t)__builtin_ctz(hits);
+        else slot = m1 & 7u;
+        st.cur = w1.x + slot;
+        hits &= ~(1u << slot);
+        if (hits) {
+            // (a negative t_min, whose keys do not order as integers, makes
+            // the bound a NaN: nothing is skipped)
+            const uint32_t bound = ANY ? 0u : (m2 & 0xFFFF0000u) | (tmin < 0.0f ? 0xFFFF0000u : 0u);
+            if (!wide_push<LDS_STACK>(st, ws, u32x2{w1.x | (neg ? kDescend : 0u), bound | hits})) return kStepFallback;
+        }
+    }
+    return kStepContinue;
+}
+
+// One node step (tg_mask == 0): visits st.cur, or the next child of the
+// stack's top group (entering or leaving an instance: INST).  Returns
+// kStepContinue, kStepDone when nothing is left (result ready for
+// wide_finish), or kStepFallback when the stack is exhausted (the exact engine
+// answers).  world_ray(o, d): the query's world ray, for leaving an instance
+// (a functor, so that only that reads it).
+template <int LDS_STACK, bool ANY, bool WT = false, bool INST = false, class WorldRay>
+VR_HD int wide_node_step(const SceneView& sv, WideState& st, const WideStack& ws, float tmin, float tmax_any,
+                         WorldRay world_ray) {
+    while (st.cur == kNoNode) {
+        if (st.sp == 0) return kStepDone;
+        const u32x2 e = wide_top<LDS_STACK>(st, ws);
+        if (INST && (e.x & kInstEntry)) {
+            --st.sp;
+            if (e.x == kInstExit) {
+                vf3 wo, wd;
+                world_ray(wo, wd);
+                wide_instance_exit<WT>(st, wo, wd);
+            } else if (ANY || !(u2f(e.y) > st.tbest * kCullSlack)) {  // (else the box lies beyond the best hit)
+                return wide_instance_enter<LDS_STACK, WT>(sv, st, ws, e.x, tmin);
+            }
+            continue;
+        }
+        if (!ANY && u2f(e.y & 0xFFFF0000u) > st.tbest * kCullSlack) {
+            --st.sp;
+            continue;
+        }
+        const uint32_t hits = e.y & 0xFFu;
+        const uint32_t slot = (e.x & kDescend) ? 31u - (uint32_t)__builtin_clz(hits) : (uint32_t)__builtin_ctz(hits);
+        st.cur = (e.x & ~kDescend) + slot;
+        if (hits & (hits - 1u)) wide_set_top<LDS_STACK>(st, ws, u32x2{e.x, e.y & ~(1u << slot)});
+        else --st.sp;
+    }
+    const uint32_t node = st.cur;
+    return wide_node<LDS_STACK, ANY>(sv, st, ws, node, tmin, tmax_any);
 }
 
 // Result of a finished query (after kStepDone).  Returns kStepDone or
@@ -564,8 +622,13 @@ VR_HD int trace_wide(const SceneView& sv, vf3 o, vf3 d, float tmin, float tmax_a
     wide_init<WT>(st, o, d, sv.num_qnodes > 0);
     if (sv.num_analytic) wide_seed_analytic<ANY, WT>(sv, st, tmin, tmax_any);
     int rc;
-    while ((rc = wide_step<LDS_STACK, ANY, WT, INST>(sv, st, ws, tmin, tmax_any, o, d)) == kStepContinue) {
-    }
+    do {
+        rc = st.tg_mask ? wide_tri_step<LDS_STACK, ANY, WT, INST>(sv, st, ws, tmin, tmax_any)
+                        : wide_node_step<LDS_STACK, ANY, WT, INST>(sv, st, ws, tmin, tmax_any, [&](vf3& wo, vf3& wd) {
+                              wo = o;
+                              wd = d;
+                          });
+    } while (rc == kStepContinue);
     if (rc == kStepFallback) {
         out.prim = 0xFFFFFFFFu;
         return kStepFallback;
