@@ -114,6 +114,23 @@ struct alignas(16) AnalyticDev {
     uint32_t surface, prim;
 };
 
+// What shading a hit needs of its prim, in one 32-byte read: the vertices
+// (indices into SceneView::verts), the material of the prim's surface and the
+// face normal.  (Through prim -> surface -> mesh -> indices these were four
+// dependent reads from as many arrays.)
+struct alignas(16) PrimRec {
+    uint32_t v[3];
+    uint32_t material;
+    float fn[3];                 // mesh.rs:80-84; object space for an instance
+    int32_t special;             // kPrimMesh, kPrimAnalytic | analytic index, or the instance's index
+};
+static_assert(sizeof(PrimRec) == 32, "PrimRec must be 32 bytes");
+constexpr int32_t kPrimMesh = -1, kPrimAnalytic = 0x40000000;
+struct alignas(16) VertRec {
+    float n[3], u, v, pad[3];
+};
+static_assert(sizeof(VertRec) == 32, "VertRec must be 32 bytes");
+
 struct GpuMaterial {
     int32_t kind;
     float color[3];
@@ -142,11 +159,9 @@ struct SceneView {
     const MeshInfo* meshes;
     const SurfaceInfo* surfaces;
     const uint32_t* mesh_idx;     // per mesh triangle: 3 vertex indices (mesh-local)
-    const float* face_n;          // per mesh triangle: face normal (mesh.rs:80-84)
     const float* vpos;            // concatenated vertices
-    const float* vnrm;
-    const float* vuv;
-    const uint32_t* prim_surface; // global prim -> surface
+    const VertRec* verts;         // concatenated vertices: normal and uv
+    const PrimRec* prims;         // per global prim
     const int32_t* ref_parent;    // per ref node: parent ref node, -1 at a mesh root
     const int32_t* prim_anc;      // global prim -> parent of its leaf in the mesh tree (-1: none)
     const AnalyticDev* analytic;  // analytic surfaces, in surface order
@@ -216,13 +231,15 @@ struct HostScene {
     std::vector<TriRec> tris;
     std::vector<uint32_t> tri_ref;  // leaf order -> tris index; empty: tris are in leaf order
     std::vector<RefNode> ref_nodes, top_nodes;
-    std::vector<uint32_t> top_path, mesh_idx, prim_surface;
+    std::vector<uint32_t> top_path, mesh_idx;
+    std::vector<VertRec> verts;
+    std::vector<PrimRec> prims;
     std::vector<int32_t> ref_parent, prim_anc, mesh_leaf_parent;
     std::vector<MeshInfo> meshes;
     std::vector<SurfaceInfo> surfaces;
     std::vector<AnalyticDev> analytic;
     std::vector<InstanceDev> instances;
-    std::vector<float> face_n, vpos, vnrm, vuv, env, env_marg, env_cond, env_pdf;
+    std::vector<float> vpos, env, env_marg, env_cond, env_pdf;
     std::vector<uint32_t> env_marg_guide, env_cond_guide;
     std::vector<GpuMaterial> materials;
     std::vector<GpuTexture> textures;

@@ -321,8 +321,11 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
     const uint32_t stride = gridDim.x * blockDim.x;
     // the same trip count for every thread of the block, so that all of them
     // reach the block-wide appends
-    for (uint32_t kb = blockIdx.x * blockDim.x; kb < n; kb += stride) {
-        uint32_t k = kb + threadIdx.x;
+    // Few live paths: the waves take theirs across all blocks (and CUs) instead
+    // of filling the first ones; a path is a chain of about ten dependent reads.
+    const bool spread = n <= stride;
+    for (uint32_t kb = spread ? 0u : blockIdx.x * blockDim.x; kb < n; kb += stride) {
+        uint32_t k = spread ? ((threadIdx.x >> 6) * gridDim.x + blockIdx.x) * 64u + (threadIdx.x & 63u) : kb + threadIdx.x;
         bool act = k < n;
         uint32_t p = 0;
         bool cont = false, shadow = false, miss = false, textured = false, env_is = false;
@@ -360,7 +363,7 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                 }
             } else {
                 HitRec hit = make_hit(sv, o, d, prim, a.hit_t[p], a.hit_u[p], a.hit_v[p]);
-                GpuMaterial m = sv.materials[sv.surfaces[hit.surface].material];
+                GpuMaterial m = sv.materials[hit.material];
                 textured = m.albedo_tex >= 0 || m.normal_tex >= 0;
                 if (!ext) {
                     if (r.mode == VR_MODE_NORMAL) {
@@ -368,7 +371,9 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                         vf3 att = mk3(0.5f * nn.x + 0.5f, 0.5f * nn.y + 0.5f, 0.5f * nn.z + 0.5f);
                         st3(a.L, p, fold_levels(a, p, depth, mk3(0.f, 0.f, 0.f) + vminc(att, c), c));
                     } else {
-                        ScatterOut sc = scatter<MICRO>(sv, m, d, hit, rng, capped, false);
+                        LambertSurf ls{};
+                        if (m.kind == VR_MAT_LAMBERTIAN) ls = lambert_surf(sv, m, hit);
+                        ScatterOut sc = scatter<MICRO>(sv, m, ls, d, hit, rng, capped, false);
                         if (!sc.has_ray) {
                             st3(a.L, p, fold_levels(a, p, depth, mk3(0.f, 0.f, 0.f) + vminc(sc.att, c), c));
                         } else {
@@ -389,9 +394,15 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                         train_hash(a.path_pix[p], a.path_smp[p], r.request, r.frame) < r.train_threshold;
                     const bool query = CACHE && r.cmode == kCacheOn && !train_path && depth >= r.cache_depth &&
                                        cache_roughness(m) >= r.query_roughness;
+                    // a Lambertian's textures, read once for the record, next-event
+                    // estimation and scattering
+                    LambertSurf ls{};
+                    if (m.kind == VR_MAT_LAMBERTIAN && !query) ls = lambert_surf(sv, m, hit);
                     if (query || (train_path && depth < r.train_vertices)) {
                         // the vertex, its outgoing direction and the path state before its contributions
-                        vf3 ns = m.normal_tex >= 0 ? tex_sample(sv, m.normal_tex, hit.uv.x, hit.uv.y) : hit.normal;
+                        vf3 ns = m.kind == VR_MAT_LAMBERTIAN && !query ? ls.n
+                                 : m.normal_tex >= 0 ? tex_sample(sv, m.normal_tex, hit.uv.x, hit.uv.y)
+                                                     : hit.normal;
                         rec = query ? 2u : 1u;
                         rec_pos = hit.point;
                         rec_dir = -d;
@@ -409,8 +420,7 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                             sv.env_kind == VR_ENV_HDRI) {
                             // next-event estimation towards the environment
                             float u1 = rng.uniform(), u2 = rng.uniform();
-                            vf3 ns = m.normal_tex >= 0 ? tex_sample(sv, m.normal_tex, hit.uv.x, hit.uv.y) : hit.normal;
-                            ns = normalize3(ns);
+                            vf3 ns = normalize3(ls.n);
                             float pe = 0.f;
                             vf3 wi = env_sample_dir(sv, u1, u2, pe);
                             env_is = true;
@@ -418,16 +428,14 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                             if (cw > 0.f && pe > 0.f) {
                                 float pb = cw / kPi;
                                 float w = (pe * pe) / (pe * pe + pb * pb);
-                                vf3 albedo = m.albedo_tex >= 0 ? tex_sample(sv, m.albedo_tex, hit.uv.x, hit.uv.y)
-                                                               : mk3(m.color[0], m.color[1], m.color[2]);
-                                vf3 contrib = mulv(mulv(A, albedo), env_lookup(sv, wi)) * (pb * w / pe);
+                                vf3 contrib = mulv(mulv(A, ls.albedo), env_lookup(sv, wi)) * (pb * w / pe);
                                 st3(a.sh_o, p, hit.point);
                                 st3(a.sh_d, p, wi);
                                 st3(a.sh_c, p, contrib);
                                 shadow = true;
                             }
                         }
-                        ScatterOut sc = scatter<MICRO>(sv, m, d, hit, rng, capped, true);
+                        ScatterOut sc = scatter<MICRO>(sv, m, ls, d, hit, rng, capped, true);
                         if (sc.has_ray && !last) {
                             A = mulv(A, sc.att);
                             float pb = 0.f;
@@ -528,17 +536,50 @@ __global__ void k_cache_mark(uint32_t* count) {
 }
 
 // Per pixel: sum of the samples in index order, scaled by 1/total_samples
-// and added into the request's target (iterative.rs:45-51).
-__global__ void k_accumulate(RenderArgs a) {
-    uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= a.npix) return;
-    uint32_t k = seg_find(a.segs, a.nseg, q, [](const SegDev& s) { return s.pix_base; });
+// and added into the request's target (iterative.rs:45-51).  A pixel's samples
+// are consecutive, so one lane per pixel reads 12 bytes out of every
+// 12 * spp: with more than a few samples a wave stages 16 samples of its 64
+// pixels in LDS (read in runs of 192 bytes, rows of 49 words against bank
+// conflicts) and each lane sums its row.  64 spp at 1080p: 2.04 ms without.
+constexpr int kAccBlock = 256, kAccSamples = 16, kAccRow = 3 * kAccSamples + 1;
+__global__ __launch_bounds__(kAccBlock) void k_accumulate(RenderArgs a) {
+    __shared__ float tile[kAccBlock / 64][64 * kAccRow];
+    const uint32_t q = blockIdx.x * kAccBlock + threadIdx.x, lane = threadIdx.x & 63u;
+    const bool act = q < a.npix;
+    const uint32_t k = seg_find(a.segs, a.nseg, act ? q : a.npix - 1u, [](const SegDev& s) { return s.pix_base; });
     const SegDev sg = a.segs[k];
     const ReqDev& r = a.reqs[sg.req];
-    uint32_t local = q - sg.pix_base;
-    uint32_t base = sg.path_base + local * r.spp;
+    const uint32_t local = q - sg.pix_base, spp = r.spp;
+    const uint32_t base = sg.path_base + local * spp;
     vf3 color = mk3(0.f, 0.f, 0.f);
-    for (uint32_t s = 0; s < r.spp; ++s) color = color + ld3(a.L, base + s);
+    // (the whole wave, and one request: a pixel's samples follow its neighbour's)
+    if (spp > 4u && __all(act && k == (uint32_t)__builtin_amdgcn_readfirstlane((int)k))) {
+        float* t = tile[threadIdx.x >> 6];
+        const float* src = a.L + 3 * (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        for (uint32_t s0 = 0; s0 < spp; s0 += kAccSamples) {
+            const uint32_t ns = min(spp - s0, (uint32_t)kAccSamples);
+            float v[3 * kAccSamples];
+#pragma unroll
+            for (int i = 0; i < 3 * kAccSamples; ++i) {
+                const uint32_t e = (uint32_t)i * 64u + lane, px = e / (3u * kAccSamples), f = e % (3u * kAccSamples);
+                v[i] = f < 3u * ns ? src[3 * ((size_t)px * spp + s0) + f] : 0.f;
+            }
+            __builtin_amdgcn_wave_barrier();  // the rows of the round before have been summed
+#pragma unroll
+            for (int i = 0; i < 3 * kAccSamples; ++i) {
+                const uint32_t e = (uint32_t)i * 64u + lane, px = e / (3u * kAccSamples), f = e % (3u * kAccSamples);
+                t[px * kAccRow + f] = v[i];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const float* row = t + lane * kAccRow;
+            for (uint32_t s = 0; s < ns; ++s) color = color + mk3(row[3 * s], row[3 * s + 1], row[3 * s + 2]);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    } else if (act) {
+        for (uint32_t s = 0; s < spp; ++s) color = color + ld3(a.L, base + s);
+    }
+    if (!act) return;
     color = color * (1.0f / (float)r.total);
     float* t = r.rgba + 4 * (size_t)(sg.pix0 + local);
     if (r.flags & VR_RENDER_OVERWRITE) {
@@ -1044,7 +1085,7 @@ static int enqueue_batch(vr_ctx* ctx, hipStream_t st) {
                     hipLaunchKernelGGL(k_cache_apply, dim3(grid_for(c.npaths, sb)), dim3(sb), 0, st, a);
                     hipLaunchKernelGGL(k_cache_targets, dim3(grid_for(c.npaths, sb)), dim3(sb), 0, st, a);
                 }
-                hipLaunchKernelGGL(k_accumulate, dim3((c.npix + sb - 1) / sb), dim3(sb), 0, st, a);
+                hipLaunchKernelGGL(k_accumulate, dim3((c.npix + kAccBlock - 1) / kAccBlock), dim3(kAccBlock), 0, st, a);
                 hipLaunchKernelGGL(k_stats_chunk, dim3(1), dim3(64), 0, st, (const uint32_t*)a.cnt, R.stats_dev,
                                    c.npaths, g.max_depth);
             }

@@ -8,8 +8,9 @@
 //                                         one record per leaf holding a piece of a split triangle)
 //   ref/top  RefNode[]              32 B  reference median-split trees (exact engine)
 //   ref_parent, prim_anc            4 B   reference-tree parents, per prim its leaf's parent
-//   per mesh triangle: idx (12 B), face normal (12 B)
-//   per vertex: position, normal (12 B each), uv (8 B)
+//   per mesh triangle: idx (12 B); per vertex: position (12 B)
+//   verts    VertRec[]              32 B  per vertex: normal, uv (shading)
+//   prims    PrimRec[T]             32 B  per prim: vertices, material, face normal (shading)
 //   materials, textures (RGBA8 or RGB f32 texels), HDRI (RGB f32) + IS tables
 #include <algorithm>
 #include <chrono>
@@ -88,7 +89,9 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
     uint32_t M = d->num_meshes;
     std::vector<MeshInfo>& minfo = H.meshes;
     minfo.assign(M, MeshInfo{});
-    std::vector<float>&vpos = H.vpos, &vnrm = H.vnrm, &vuv = H.vuv, &face_n = H.face_n;
+    std::vector<float>& vpos = H.vpos;
+    std::vector<float> face_n;  // per mesh triangle (mesh.rs:80-84)
+    std::vector<VertRec>& verts = H.verts;
     std::vector<uint32_t>& midx = H.mesh_idx;
     std::vector<RefNode>& ref_nodes = H.ref_nodes;
     std::vector<int32_t>&ref_parent = H.ref_parent, &leaf_parent = H.mesh_leaf_parent;
@@ -100,8 +103,7 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
     }
     if (tv >= (1ull << 32) || tt >= (1ull << 31)) return fail(VR_ERR_INVALID, "scene too large");
     vpos.reserve(3 * tv);
-    vnrm.reserve(3 * tv);
-    vuv.reserve(2 * tv);
+    verts.reserve(tv);
     midx.reserve(3 * tt);
     face_n.reserve(3 * tt);
     for (uint32_t m = 0; m < M; ++m) {
@@ -115,12 +117,14 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
         mi.root = -1;
         Box3 mb{mk3(kInf, kInf, kInf), mk3(-kInf, -kInf, -kInf)};  // AABB::default
         for (uint32_t i = 0; i < src.num_vertices; ++i) {
+            VertRec vr{};
             for (int a = 0; a < 3; ++a) {
                 vpos.push_back(src.positions[3 * i + a]);
-                vnrm.push_back(src.normals ? src.normals[3 * i + a] : 0.0f);
+                vr.n[a] = src.normals ? src.normals[3 * i + a] : 0.0f;
             }
-            vuv.push_back(src.uvs ? src.uvs[2 * i] : 0.0f);
-            vuv.push_back(src.uvs ? src.uvs[2 * i + 1] : 0.0f);
+            vr.u = src.uvs ? src.uvs[2 * i] : 0.0f;
+            vr.v = src.uvs ? src.uvs[2 * i + 1] : 0.0f;
+            verts.push_back(vr);
             vf3 p = ld3(src.positions, i);
             mb.lo = mk3(fminf(mb.lo.x, p.x), fminf(mb.lo.y, p.y), fminf(mb.lo.z, p.z));
             mb.hi = mk3(fmaxf(mb.hi.x, p.x), fmaxf(mb.hi.y, p.y), fmaxf(mb.hi.z, p.z));
@@ -316,18 +320,31 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
     // ---- fast structure: triangle records + SAH quantised BVH4 ------------
     std::vector<TriRec> recs;
     recs.reserve(T);
-    std::vector<uint32_t>& prim_surface = H.prim_surface;
-    prim_surface.assign(T, 0);
+    std::vector<PrimRec>& prims = H.prims;
+    prims.assign(T, PrimRec{});
+    auto fill_prims = [&](uint32_t i, int32_t special) {  // the triangles of surface i
+        const MeshInfo& mi = minfo[sinfo[i].mesh];
+        for (uint32_t t = 0; t < mi.num_tris; ++t) {
+            PrimRec& p = prims[sinfo[i].prim_base + t];
+            for (int a = 0; a < 3; ++a) {
+                p.v[a] = mi.vert_base + midx[3 * (size_t)(mi.tri_base + t) + a];
+                p.fn[a] = face_n[3 * (size_t)(mi.tri_base + t) + a];
+            }
+            p.material = sinfo[i].material;
+            p.special = special;
+        }
+    };
     std::vector<int32_t>& prim_anc = H.prim_anc;
     prim_anc.assign(T, -1);
     for (uint32_t i = 0; i < S; ++i) {
         if (sinfo[i].analytic >= 0) {  // not in the wide BVH: tested per ray (traverse.h)
-            prim_surface[sinfo[i].prim_base] = i;
+            prims[sinfo[i].prim_base].material = sinfo[i].material;
+            prims[sinfo[i].prim_base].special = kPrimAnalytic | sinfo[i].analytic;
             continue;
         }
         if (sinfo[i].instance >= 0) {  // one top-level entry: the instance's world box
             const MeshInfo& mi = minfo[sinfo[i].mesh];
-            for (uint32_t t = 0; t < mi.num_tris; ++t) prim_surface[sinfo[i].prim_base + t] = i;
+            fill_prims(i, sinfo[i].instance);
             if (mi.num_tris == 0) continue;
             recs.emplace_back();
             TriRec& r = recs.back();
@@ -349,6 +366,7 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
             continue;
         }
         const MeshInfo& mi = minfo[sinfo[i].mesh];
+        fill_prims(i, kPrimMesh);
         for (uint32_t t = 0; t < mi.num_tris; ++t) {
             recs.emplace_back();
             TriRec& r = recs.back();
@@ -367,7 +385,6 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
                 xb = 0x7FC00000u;
                 std::memcpy(&r.p2[0], &xb, 4);
             }
-            prim_surface[sinfo[i].prim_base + t] = i;
             prim_anc[sinfo[i].prim_base + t] = leaf_parent[mi.tri_base + t];
         }
     }
@@ -524,11 +541,9 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
     v.meshes = minfo.data();
     v.surfaces = sinfo.data();
     v.mesh_idx = midx.data();
-    v.face_n = face_n.data();
     v.vpos = vpos.data();
-    v.vnrm = vnrm.data();
-    v.vuv = vuv.data();
-    v.prim_surface = prim_surface.data();
+    v.verts = verts.data();
+    v.prims = prims.data();
     v.ref_parent = ref_parent.data();
     v.prim_anc = prim_anc.data();
     v.analytic = analytic.data();
@@ -581,11 +596,9 @@ int build_scene(vr_ctx* ctx, const vr_scene_desc* d, vr_scene* s) {
     rc |= upload(s, H.meshes, &v.meshes);
     rc |= upload(s, H.surfaces, &v.surfaces);
     rc |= upload(s, H.mesh_idx, &v.mesh_idx);
-    rc |= upload(s, H.face_n, &v.face_n);
     rc |= upload(s, H.vpos, &v.vpos);
-    rc |= upload(s, H.vnrm, &v.vnrm);
-    rc |= upload(s, H.vuv, &v.vuv);
-    rc |= upload(s, H.prim_surface, &v.prim_surface);
+    rc |= upload(s, H.verts, &v.verts);
+    rc |= upload(s, H.prims, &v.prims);
     rc |= upload(s, H.ref_parent, &v.ref_parent);
     rc |= upload(s, H.prim_anc, &v.prim_anc);
     rc |= upload(s, H.analytic, &v.analytic);

@@ -15,10 +15,18 @@ VR_HD uint64_t as_usize(float x) {
     return (uint64_t)x;
 }
 
+// b / 255 for a byte b, rounded once: the product with the rounded reciprocal,
+// corrected by its remainder (equal to the division for all 256 values).
+VR_HD float unorm8(uint32_t b) {
+    const float x = (float)b, r = 1.0f / 255.0f;
+    const float q = x * r;
+    return fmaf(fmaf(-q, 255.0f, x), r, q);
+}
+
 VR_HD vf3 texel(const SceneView& sv, const GpuTexture& t, uint64_t i) {
     if (t.format == VR_TEX_RGBA8) {
-        const uint8_t* p = sv.tex_data + t.offset + 4 * i;
-        return mk3((float)p[0] / 255.0f, (float)p[1] / 255.0f, (float)p[2] / 255.0f);
+        const uint32_t p = *(const uint32_t*)(sv.tex_data + t.offset + 4 * i);  // (offsets are multiples of 256)
+        return mk3(unorm8(p & 0xFFu), unorm8((p >> 8) & 0xFFu), unorm8((p >> 16) & 0xFFu));
     }
     const float* p = (const float*)(sv.tex_data + t.offset) + 3 * i;
     return mk3(p[0], p[1], p[2]);
@@ -37,8 +45,16 @@ VR_HD vf3 bilinear(uint32_t W, uint32_t H, float x, float y, Fetch fetch) {
     if (y0 > H - 1) y0 = H - 1;
     float ax = x - (float)x0;
     float ay = y - (float)y0;
-    return lerp3(lerp3(fetch((y0 * W + x0) % len), fetch((y0 * W + x0 + 1) % len), ax),
-                 lerp3(fetch(((y0 + 1) * W + x0) % len), fetch(((y0 + 1) * W + x0 + 1) % len), ax), ay);
+    // The texels (y0 W + x0, + 1, + W, + W + 1) % len.  With x0 < W and y0 < H the
+    // first is below len and the last below len + W + 1 <= 2 len + 1, so
+    // subtracting len at most twice gives the remainder without a division
+    // (a 64-bit modulo is over a hundred instructions, and there were four).
+    auto wrap = [&](uint64_t i) {
+        i = i >= len ? i - len : i;
+        return i >= len ? i - len : i;
+    };
+    const uint64_t i0 = y0 * W + x0;
+    return lerp3(lerp3(fetch(i0), fetch(wrap(i0 + 1)), ax), lerp3(fetch(wrap(i0 + W)), fetch(wrap(i0 + W + 1)), ax), ay);
 }
 
 // Rust's x % 1.0 (fmod(x, 1)): x - trunc(x), which is exact, with the sign
@@ -56,7 +72,7 @@ VR_HD vf3 tex_sample(const SceneView& sv, int32_t ti, float u, float v) {
         uint64_t xi = as_usize(x), yi = as_usize(y);
         if (xi > t.w - 1) xi = t.w - 1;
         if (yi > t.h - 1) yi = t.h - 1;
-        return texel(sv, t, (yi * t.w + xi) % ((uint64_t)t.w * t.h));
+        return texel(sv, t, yi * t.w + xi);  // (below w h: no wrap)
     }
     return bilinear(t.w, t.h, x, y, [&](uint64_t i) { return texel(sv, t, i); });
 }
@@ -292,45 +308,40 @@ struct HitRec {
     vf3 point, normal;
     vf2 uv;
     bool front;
-    uint32_t surface;
+    uint32_t material;
 };
 
 VR_HD HitRec make_hit(const SceneView& sv, vf3 o, vf3 d, uint32_t prim, float t, float u, float v) {
     HitRec h;
-    uint32_t surf = sv.prim_surface[prim];
-    SurfaceInfo si = sv.surfaces[surf];
-    if (si.analytic >= 0) {
+    const PrimRec pr = sv.prims[prim];
+    h.material = pr.material;
+    if (pr.special >= kPrimAnalytic) {
         // Sphere::hit / GroundPlane::hit hit records (surfaces.rs:71-77, 96-103):
         // outward normal (point - centre) / radius or +y; u, v carry the uv
-        const AnalyticDev& a = sv.analytic[si.analytic];
+        const AnalyticDev& a = sv.analytic[pr.special & ~kPrimAnalytic];
         h.point = o + d * t;
         vf3 n = a.kind == VR_ANALYTIC_SPHERE ? (h.point - mk3(a.c[0], a.c[1], a.c[2])) / a.r : mk3(0.f, 1.f, 0.f);
         h.uv.x = u;
         h.uv.y = v;
         h.front = dot3(d, n) < 0.0f;
         h.normal = h.front ? n : -n;
-        h.surface = surf;
         return h;
     }
-    MeshInfo mi = sv.meshes[si.mesh];
-    uint32_t tri = prim - si.prim_base;
-    const uint32_t* ix = sv.mesh_idx + 3 * (size_t)(mi.tri_base + tri);
-    size_t v0 = mi.vert_base + ix[0], v1 = mi.vert_base + ix[1], v2 = mi.vert_base + ix[2];
-    vf3 n0 = mk3(sv.vnrm[3 * v0], sv.vnrm[3 * v0 + 1], sv.vnrm[3 * v0 + 2]);
-    vf3 n1 = mk3(sv.vnrm[3 * v1], sv.vnrm[3 * v1 + 1], sv.vnrm[3 * v1 + 2]);
-    vf3 n2 = mk3(sv.vnrm[3 * v2], sv.vnrm[3 * v2 + 1], sv.vnrm[3 * v2 + 2]);
+    const VertRec a0 = sv.verts[pr.v[0]], a1 = sv.verts[pr.v[1]], a2 = sv.verts[pr.v[2]];
+    vf3 n0 = mk3(a0.n[0], a0.n[1], a0.n[2]);
+    vf3 n1 = mk3(a1.n[0], a1.n[1], a1.n[2]);
+    vf3 n2 = mk3(a2.n[0], a2.n[1], a2.n[2]);
     float w = (1.0f - u) - v;
     // Triangle::hit shading (mesh.rs:176-181)
     vf3 n = (u * n1 + v * n2) + w * n0;
-    h.uv.x = (u * sv.vuv[2 * v1] + v * sv.vuv[2 * v2]) + w * sv.vuv[2 * v0];
-    h.uv.y = (u * sv.vuv[2 * v1 + 1] + v * sv.vuv[2 * v2 + 1]) + w * sv.vuv[2 * v0 + 1];
-    const float* fp = sv.face_n + 3 * (size_t)(mi.tri_base + tri);
-    vf3 fn = mk3(fp[0], fp[1], fp[2]);
-    if (si.instance >= 0) {
+    h.uv.x = (u * a1.u + v * a2.u) + w * a0.u;
+    h.uv.y = (u * a1.v + v * a2.v) + w * a0.v;
+    vf3 fn = mk3(pr.fn[0], pr.fn[1], pr.fn[2]);
+    if (pr.special >= 0) {
         // an instance's mesh holds object-space normals: n' = (M^-1)^T n; the
         // face normal of the placed triangle is that of its object-space
         // normal, flipped when M reverses the winding
-        const InstanceDev& x = sv.instances[si.instance];
+        const InstanceDev& x = sv.instances[pr.special];
         const float* q = x.nrm;
         n = mk3((q[0] * n.x + q[1] * n.y) + q[2] * n.z, (q[3] * n.x + q[4] * n.y) + q[5] * n.z,
                 (q[6] * n.x + q[7] * n.y) + q[8] * n.z);
@@ -344,8 +355,19 @@ VR_HD HitRec make_hit(const SceneView& sv, vf3 o, vf3 d, uint32_t prim, float t,
     h.point = o + d * t;
     h.front = dot3(d, n) < 0.0f;
     h.normal = h.front ? n : -n;
-    h.surface = surf;
     return h;
+}
+
+// A Lambertian's normal (its map's or the hit's) and albedo at a hit.
+struct LambertSurf {
+    vf3 n, albedo;
+};
+VR_HD LambertSurf lambert_surf(const SceneView& sv, const GpuMaterial& m, const HitRec& hit) {
+    LambertSurf s;
+    s.n = m.normal_tex >= 0 ? tex_sample(sv, m.normal_tex, hit.uv.x, hit.uv.y) : hit.normal;
+    s.albedo = m.albedo_tex >= 0 ? tex_sample(sv, m.albedo_tex, hit.uv.x, hit.uv.y)
+                                 : mk3(m.color[0], m.color[1], m.color[2]);
+    return s;
 }
 
 struct ScatterOut {
@@ -360,23 +382,22 @@ struct ScatterOut {
 // `cosine_lobe`: the extended estimator's Lambertian, which scatters about the
 // normalised shading normal so that its pdf is cos/pi exactly.  MICRO: the
 // scene has MicrofacetBSDF materials (compiled out otherwise: the caller
-// only passes false for scenes without them).
+// only passes false for scenes without them).  ls: lambert_surf of a Lambertian.
 template <bool MICRO = true>
-VR_HD ScatterOut scatter(const SceneView& sv, const GpuMaterial& m, vf3 d, const HitRec& hit, PathRng& rng,
-                         uint32_t& capped, bool cosine_lobe) {
+VR_HD ScatterOut scatter(const SceneView& sv, const GpuMaterial& m, const LambertSurf& ls, vf3 d, const HitRec& hit,
+                         PathRng& rng, uint32_t& capped, bool cosine_lobe) {
     ScatterOut s;
     s.diffuse = false;
     s.lobe = mk3(0.f, 0.f, 0.f);
     switch (m.kind) {
         case VR_MAT_LAMBERTIAN: {
-            vf3 n = m.normal_tex >= 0 ? tex_sample(sv, m.normal_tex, hit.uv.x, hit.uv.y) : hit.normal;
+            vf3 n = ls.n;
             if (cosine_lobe) n = normalize3(n);
             vf3 dir = n + unit_sphere(rng, capped);
             if (near_zero(dir)) dir = n;
             s.dir = normalize3(dir);
             s.has_ray = true;
-            s.att = m.albedo_tex >= 0 ? tex_sample(sv, m.albedo_tex, hit.uv.x, hit.uv.y)
-                                      : mk3(m.color[0], m.color[1], m.color[2]);
+            s.att = ls.albedo;
             s.diffuse = true;
             s.lobe = n;
             return s;
