@@ -27,6 +27,12 @@ constexpr int kRefillAny = 32;
 // 7% slower).
 constexpr int kVote = 3;
 constexpr int kVoteAny = 2;
+// Up to this many rays per launched wave go eight lanes to a ray, two to a
+// group (trace_groups).  64 rays: 45 -> 31 us; a 960 x 540 x 4 frame, whose late
+// bounces hold a few thousand rays, 6.49 -> 5.80 ms; 16 requests of mixed sizes
+// 57.7 -> 51.9 ms.  With 4, 8 and 32 rays a wave the reference-estimator frame
+// (719p x 8) took 7.13, 6.93 and 7.17 ms instead of 6.93.
+constexpr uint32_t kGroupRays = 16;
 
 struct TraceArgs {
     SceneView sv;  // first (cold_args)
@@ -114,6 +120,247 @@ constexpr int kFetchStride = 32;  // words between two partition counters
 static_assert(kCtrFetch + kFetchParts * kFetchStride <= kCtrWords, "counter block too small");
 static_assert(kFetchParts <= 64, "one lane clears each partition counter");
 
+// ---- few rays: eight lanes a ray --------------------------------------------
+// A launch with few rays takes as long as its longest ray's chain of steps, and
+// a step of one lane is about 270 dependent-issue instructions besides its
+// memory latency.  Eight lanes share a ray instead: each tests one child box of
+// a node, or one record of the node's leaves (all of them, whichever leaf was
+// hit: a superset of the candidates changes no answer), and the results meet
+// in cross-lane reductions.  All lanes of a group hold the same state and make
+// the same branches.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xF, 0xF, true);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141;  // lane ^ 1, ^ 2, 7 - lane of each 8
+// Minimum over the 8 lanes of a group.
+__device__ __forceinline__ uint32_t min8_u(uint32_t x) {
+    x = min(x, dpp_u<kDppXor1>(x));
+    x = min(x, dpp_u<kDppXor2>(x));
+    return min(x, dpp_u<kDppHalfMirror>(x));
+}
+__device__ __forceinline__ float min8_f(float x) {
+    x = fminf(x, u2f(dpp_u<kDppXor1>(f2u(x))));
+    x = fminf(x, u2f(dpp_u<kDppXor2>(f2u(x))));
+    return fminf(x, u2f(dpp_u<kDppHalfMirror>(f2u(x))));
+}
+
+// Node step of a group (as wide_node_step and wide_node; `stk`: the group's
+// stack in LDS, CAP entries; every lane writes the same entry).
+template <int CAP, bool ANY, bool WT, bool INST, class WorldRay>
+__device__ __forceinline__ uint32_t group_node_step(const SceneView& sv, WideState& st, lds_u32x2* stk, uint32_t c,
+                                                    float tmin, float tmax_any, WorldRay world_ray) {
+    while (st.cur == kNoNode) {
+        if (st.sp == 0) return kStepDone;
+        const u32x2 e = stk[st.sp - 1];
+        if (INST && (e.x & kInstEntry)) {
+            --st.sp;
+            if (e.x == kInstExit) {
+                vf3 wo, wd;
+                world_ray(wo, wd);
+                wide_instance_exit<WT>(st, wo, wd);
+            } else if (ANY || !(u2f(e.y) > st.tbest * kCullSlack)) {
+                if (st.sp >= CAP) return kStepFallback;
+                const WideStack ws{stk, 1, nullptr, 0, 0};
+                return (uint32_t)wide_instance_enter<CAP, WT>(sv, st, ws, e.x, tmin);
+            }
+            continue;
+        }
+        if (!ANY && u2f(e.y & 0xFFFF0000u) > st.tbest * kCullSlack) {
+            --st.sp;
+            continue;
+        }
+        const uint32_t hits = e.y & 0xFFu;
+        const uint32_t slot = (e.x & kDescend) ? 31u - (uint32_t)__builtin_clz(hits) : (uint32_t)__builtin_ctz(hits);
+        st.cur = (e.x & ~kDescend) + slot;
+        if (hits & (hits - 1u)) stk[st.sp - 1] = u32x2{e.x, e.y & ~(1u << slot)};
+        else --st.sp;
+    }
+    const QNode* q = sv.qnodes + st.cur;
+    const u32x4 w0 = ((const u32x4*)q)[0], w1 = ((const u32x4*)q)[1];
+    const uint8_t* lo = &q->qlo[0][0] + c;  // this lane's child; hi bytes 24 after lo
+    const uint32_t lx = lo[0], ly = lo[8], lz = lo[16], hx = lo[24], hy = lo[32], hz = lo[40];
+    const uint32_t e = w0.w;
+    const float sx = u2f((e & 0xFFu) << 23) * st.idx;
+    const float sy = u2f(((e >> 8) & 0xFFu) << 23) * st.idy;
+    const float sz = u2f(((e >> 16) & 0xFFu) << 23) * st.idz;
+    const uint32_t num_inner = e >> 24;
+    const float bx = (u2f(w0.x) - st.o.x) * st.idx;
+    const float by = (u2f(w0.y) - st.o.y) * st.idy;
+    const float bz = (u2f(w0.z) - st.o.z) * st.idz;
+    const bool negx = st.idx < 0.f, negy = st.idy < 0.f, negz = st.idz < 0.f;
+    const float tcull = ANY ? tmax_any : st.tbest * kCullSlack;
+    const float nx = fmaf((float)(negx ? hx : lx), sx, bx), fx = fmaf((float)(negx ? lx : hx), sx, bx);
+    const float ny = fmaf((float)(negy ? hy : ly), sy, by), fy = fmaf((float)(negy ? ly : hy), sy, by);
+    const float nz = fmaf((float)(negz ? hz : lz), sz, bz), fz = fmaf((float)(negz ? lz : hz), sz, bz);
+    const float tnear = fmaxf(fmaxf(nx, ny), fmaxf(nz, tmin));
+    const float tfar = fminf(fminf(fx, fy), fminf(fz, tcull));
+    const bool hit = tnear <= tfar * kSlabSlack;
+    uint32_t hits = (uint32_t)(__ballot(hit) >> (threadIdx.x & 56u)) & 0xFFu;
+    const uint32_t inner = (1u << num_inner) - 1u;
+    uint32_t leaves = hits & ~inner;
+    leaves = (leaves | (leaves << 8)) & 0x00F00Fu;
+    leaves = (leaves | (leaves << 4)) & 0x0C30C3u;
+    leaves = (leaves | (leaves << 2)) & 0x249249u;
+    st.tg_all = w1.z & 0xFFFFFFu;
+    st.tg_mask = ((leaves << 3) - leaves) & st.tg_all;
+    st.tg_base = w1.y;
+    hits &= inner;
+    st.cur = kNoNode;
+    if (hits) {
+        const uint32_t axis = (w1.z >> 24) & 3u;
+        const bool neg = axis == 0u ? negx : axis == 1u ? negy : negz;
+        uint32_t slot, bound = 0;
+        if (ANY) {
+            slot = neg ? 31u - (uint32_t)__builtin_clz(hits) : (uint32_t)__builtin_ctz(hits);
+        } else {
+            const uint32_t key = hit && c < num_inner ? (f2u(tnear) & ~7u) | c : 0xFFFFFFFFu;
+            const uint32_t m1 = min8_u(key), m2 = min8_u(key == m1 ? 0xFFFFFFFFu : key);
+            slot = m1 & 7u;
+            bound = (m2 & 0xFFFF0000u) | (tmin < 0.0f ? 0xFFFF0000u : 0u);
+        }
+        st.cur = w1.x + slot;
+        hits &= ~(1u << slot);
+        if (hits) {
+            if (st.sp >= CAP) return kStepFallback;
+            stk[st.sp++] = u32x2{w1.x | (neg ? kDescend : 0u), bound | hits};
+        }
+    }
+    return kStepContinue;
+}
+
+// Record step of a group: all records of the node's leaves, eight at a time.
+template <int CAP, bool ANY, bool WT, bool INST>
+__device__ __forceinline__ uint32_t group_tri_step(const SceneView& sv, WideState& st, lds_u32x2* stk, uint32_t c,
+                                                   float tmin, float tmax_any) {
+    const uint32_t gl = threadIdx.x & 56u, count = (uint32_t)__builtin_popcount(st.tg_all);
+    const bool in_inst = INST && st.inst != kNoInstance;
+    st.tg_mask = 0;
+    for (uint32_t r0 = 0; r0 < count; r0 += 8) {
+        float t = kInf, u = 0.f, v = 0.f;
+        uint32_t prim = 0xFFFFFFFFu, slot = 0;
+        bool enter = false, found = false, unconfirmed = false;
+        u32x2 entry{};
+        if (r0 + c < count) {
+            const uint32_t rec = st.tg_base + r0 + c;
+            slot = sv.tri_ref ? sv.tri_ref[rec] : rec;
+            vf3 p0, p1, p2;
+            load_tri_geom(sv.tris, slot, p0, p1, p2);
+            if (INST && f2u(p2.x) == kInstanceMarker) {
+                const float tcull = ANY ? tmax_any : st.tbest * kCullSlack;
+                const float ax = (p0.x - st.o.x) * st.idx, bx = (p1.x - st.o.x) * st.idx;
+                const float ay = (p0.y - st.o.y) * st.idy, by = (p1.y - st.o.y) * st.idy;
+                const float az = (p0.z - st.o.z) * st.idz, bz = (p1.z - st.o.z) * st.idz;
+                const float tnear = fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fmaxf(fminf(az, bz), tmin));
+                const float tfar = fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fminf(fmaxf(az, bz), tcull));
+                enter = tnear <= tfar * kSlabSlack;
+                entry = u32x2{kInstEntry | f2u(p2.y), f2u(tnear)};
+            } else {
+                MTResult m;
+                if (WT ? wt_hit(st.wt, st.o, p0, p1, p2, tmin, m)
+                       : mt_hit(st.o, st.d, p0, p1, p2, tmin, m, in_inst ? st.inst_eps : -1.0f)) {
+                    prim = (in_inst ? st.inst_base : 0u) + tri_word(sv.tris, slot, 9);
+                    if (!ANY || m.t < tmax_any) {
+                        found = !ANY || WT || in_inst ||
+                                confirm_winner(cold_scene(sv), st.o, st.d, tmin, m.t, p0, p1, p2,
+                                               tri_word(sv.tris, slot, 11), prim);
+                        unconfirmed = !found;
+                    }
+                    t = m.t;
+                    u = m.u;
+                    v = m.v;
+                }
+            }
+        }
+        if (INST) {
+            const uint32_t es = (uint32_t)(__ballot(enter) >> gl) & 0xFFu;
+            if (es) {
+                const int ne = __builtin_popcount(es);
+                if (st.sp + ne > CAP) return kStepFallback;
+                // (lane by lane, each entry written by all lanes, as every other push)
+                for (uint32_t m = es; m; m &= m - 1u) {
+                    const int from = (int)(gl + (uint32_t)__builtin_ctz(m));
+                    stk[st.sp++] = u32x2{(uint32_t)__shfl((int)entry.x, from), (uint32_t)__shfl((int)entry.y, from)};
+                }
+            }
+        }
+        const uint32_t fs = (uint32_t)(__ballot(found) >> gl) & 0xFFu;
+        if (ANY && ((uint32_t)(__ballot(unconfirmed) >> gl) & 0xFFu)) st.unconfirmed = 1u;
+        if (fs == 0u) continue;
+        // the winner: any hit the first lane's, closest hit the least (t, prim)
+        uint32_t w;
+        if (ANY) {
+            w = (uint32_t)__builtin_ctz(fs);
+        } else {
+            const float tm = min8_f(found ? t : kInf);
+            if (tm > st.tbest) continue;
+            const bool tie = found && t == tm;
+            const uint32_t pm = min8_u(tie ? prim : 0xFFFFFFFFu);
+            if (!(tm < st.tbest || pm < st.best_prim)) continue;
+            w = (uint32_t)__builtin_ctz((uint32_t)(__ballot(tie && prim == pm) >> gl) & 0xFFu);
+        }
+        const int from = (int)(gl + w);
+        st.tbest = __shfl(t, from);
+        st.bu = __shfl(u, from);
+        st.bv = __shfl(v, from);
+        st.best_prim = (uint32_t)__shfl((int)prim, from);
+        st.best_slot = (uint32_t)__shfl((int)slot, from);
+        if (INST) st.best_inst = st.inst;
+        if (ANY) {
+            st.found = 1u;
+            return kStepDone;
+        }
+    }
+    return kStepContinue;
+}
+
+template <bool ANY, bool WT, bool INST, int LDS>
+__device__ __forceinline__ void trace_groups(const TraceArgs& a, uint32_t n, u32x2* lds) {
+    constexpr int CAP = LDS * 8;
+    const uint32_t lane = threadIdx.x, c = lane & 7u;
+    lds_u32x2* stk = (lds_u32x2*)lds + (lane >> 3) * CAP;
+    WideState st;
+    uint32_t status = kStepDone, ray = 0xFFFFFFFFu;
+    st.tg_mask = 0;
+    // one ray a wave first, then a second one, ...
+    for (uint32_t k = blockIdx.x + gridDim.x * (lane >> 3);;) {
+        if (status != kStepContinue) {
+            const TraceArgs& x = cold_args(a);
+            if (ray != 0xFFFFFFFFu) {
+                HitOut h;
+                const int rc = status == kStepFallback ? kStepFallback : wide_finish<ANY, WT, INST>(x.sv, st, x.tmin, h);
+                if (c == 0u) {
+                    if (rc == kStepFallback) x.fb_list[atomicAdd(x.fb_count, 1u)] = ray;
+                    else write_out(x, ray, h);
+                }
+                ray = 0xFFFFFFFFu;
+            }
+            if (k < n) {
+                ray = x.queue ? x.queue[k] : k;
+                k += gridDim.x * 8u;
+                status = kStepContinue;
+                const vf3 o = mk3(x.o[3 * ray], x.o[3 * ray + 1], x.o[3 * ray + 2]);
+                const vf3 d = mk3(x.d[3 * ray], x.d[3 * ray + 1], x.d[3 * ray + 2]);
+                wide_init<WT>(st, o, d, x.sv.num_qnodes > 0);
+                if (x.sv.num_analytic) wide_seed_analytic<ANY, WT>(x.sv, st, x.tmin, x.tmax);
+            }
+        }
+        const uint64_t walking = __ballot(status == kStepContinue);
+        if (walking == 0ull) break;
+        const uint64_t tri = __ballot(status == kStepContinue && st.tg_mask != 0u);
+        if (2 * __popcll(tri) >= __popcll(walking)) {
+            if (status == kStepContinue && st.tg_mask != 0u)
+                status = group_tri_step<CAP, ANY, WT, INST>(a.sv, st, stk, c, a.tmin, a.tmax);
+        } else if (status == kStepContinue && st.tg_mask == 0u) {
+            status = group_node_step<CAP, ANY, WT, INST>(a.sv, st, stk, c, a.tmin, a.tmax, [&](vf3& wo, vf3& wd) {
+                const TraceArgs& x = cold_args(a);
+                wo = mk3(x.o[3 * ray], x.o[3 * ray + 1], x.o[3 * ray + 2]);
+                wd = mk3(x.d[3 * ray], x.d[3 * ray + 1], x.d[3 * ray + 2]);
+            });
+        }
+    }
+}
+
 // Persistent wide-engine kernel: every lane runs its own ray as a resumable
 // state machine whose next step is a node or a triangle record.  In each
 // iteration the wave votes: a record step runs if enough of the walking lanes
@@ -129,6 +376,10 @@ __device__ __forceinline__ void trace_persist(const TraceArgs& a) {
     const uint32_t glane = blockIdx.x * kWave + lane;
     const WideStack ws{(lds_u32x2*)(lds + lane), kWave, a.spill + glane, (int)a.spill_lanes, a.spill_cap};
     const uint32_t n = a.count ? *a.count : a.n;
+    if (n <= gridDim.x * kGroupRays) {
+        trace_groups<ANY, WT, INST, LDS>(a, n, lds);
+        return;
+    }
     WideState st;
     uint32_t ray = 0;
     // The lane's state as one word.  (As bools they were lane masks in
