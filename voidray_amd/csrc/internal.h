@@ -264,6 +264,7 @@ struct TraceJob {
     uint32_t* prim = nullptr;
     float *t = nullptr, *u = nullptr, *v = nullptr;
     uint8_t* hit = nullptr;
+    u32x4* rec = nullptr;                // optional: {prim, t, u, v} per ray
     uint64_t* fallback_accum = nullptr;  // optional: += number of exact-engine rays
     bool timed = false;                  // record trace_ev[0..1] around the wide kernel
 };

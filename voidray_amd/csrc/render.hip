@@ -42,7 +42,7 @@ namespace vr {
 // thin them out, a small chunk leaves the traversal kernels' persistent waves
 // mostly idle.  On the 1080p x 64 spp terrain frame (132.7 M paths): 2^22
 // paths per chunk 394 ms, 2^24 215 ms, 2^26 (two chunks) 146 ms, 2^27 (one
-// chunk) 137 ms; about 133 B of path state per path with the extended
+// chunk) 137 ms; about 121 B of path state per path with the extended
 // estimator, 272 B with the reference estimator's 16-level attenuation stack:
 // 18 or 36 GB of the GPU's 288 GB at 2^27.  Scratch is sized by the largest
 // chunk a call actually uses, so small frames allocate little.
@@ -112,19 +112,20 @@ struct RenderArgs {
     const ReqDev* reqs;
     const SegDev* segs;
     uint32_t nseg, npix, npaths, cap;
-    uint32_t* path_req;
-    uint32_t* path_pix;
-    uint32_t* path_smp;
-    float* ray_o;
+    // Path state.  From the second bounce on the live paths are scattered over
+    // the chunk, so words that are read together lie together: one access per
+    // record instead of one per word, each of which moves a line of its own.
+    // Word by word, and with shadow origins of their own: cornell 512 x 512 x 16
+    // 2.76 ms instead of 2.70, the 1080p x 64 terrain 103.1 instead of 101.1.
+    uint32_t* path_id;  // [cap][3] request, pixel, sample
+    float* ray_o;       // also the origin of the path's shadow ray
     float* ray_d;
-    uint32_t* hit_prim;
-    float *hit_t, *hit_u, *hit_v;
+    u32x4* hit;  // prim, t, u, v
     uint32_t* rng_n;
     float* att;  // reference estimator: [max_bounces][cap][3]
     float* L;    // [cap][3]
-    float* A;    // extended: throughput [cap][3]
-    float* pdf;  // extended: pdf of the last diffuse scatter (0 = camera / specular)
-    float *sh_o, *sh_d, *sh_c;
+    f32x4* A;    // extended: throughput, pdf of the last diffuse scatter (0 = camera / specular)
+    float *sh_d, *sh_c;
     uint8_t* sh_hit;
     uint32_t* queue[2];
     uint32_t* sh_queue;
@@ -253,9 +254,10 @@ __global__ void k_raygen(RenderArgs a) {
     uint32_t local = p - sg.path_base;
     uint32_t i = sg.pix0 + local / r.spp;
     uint32_t s = r.sample_offset + local % r.spp;
-    a.path_req[p] = sg.req;
-    a.path_pix[p] = i;
-    a.path_smp[p] = s;
+    uint32_t* id = a.path_id + 3 * (size_t)p;
+    id[0] = sg.req;
+    id[1] = i;
+    id[2] = s;
     uint32_t W = r.W, H = r.H;
     uint32_t x = i % W;
     uint32_t y = (r.flags & VR_RENDER_ROWS_BY_HEIGHT) ? i / H : i / W;
@@ -284,10 +286,7 @@ __global__ void k_raygen(RenderArgs a) {
     st3(a.ray_d, p, dir);
     a.rng_n[p] = rng.n;
     st3(a.L, p, mk3(0.f, 0.f, 0.f));
-    if (r.ext) {
-        st3(a.A, p, mk3(1.f, 1.f, 1.f));
-        a.pdf[p] = 0.f;
-    }
+    if (r.ext) a.A[p] = f32x4{1.f, 1.f, 1.f, 0.f};
     if (capped) atomicAdd(a.cnt + kCntCapped, capped);
 }
 
@@ -335,14 +334,17 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
         uint32_t capped = 0;
         if (act) {
             p = qin ? qin[k] : k;
-            const ReqDev& r = a.reqs[a.path_req[p]];
+            const uint32_t* id = a.path_id + 3 * (size_t)p;
+            const uint32_t pix = id[1], smp = id[2];
+            const ReqDev& r = a.reqs[id[0]];
             const bool ext = EST == 2 || (EST == 0 && r.ext);
             const float c = r.clamp;
             const bool last = depth + 1 >= r.max_bounces;
             PathRng rng;
-            rng.init(r.seed, r.request, a.path_pix[p], a.path_smp[p], a.rng_n[p]);
+            rng.init(r.seed, r.request, pix, smp, a.rng_n[p]);
             vf3 o = ld3(a.ray_o, p), d = ld3(a.ray_d, p);
-            uint32_t prim = a.hit_prim[p];
+            const u32x4 hw = a.hit[p];
+            const uint32_t prim = hw.x;
             if (depth >= r.max_bounces) {
                 // max_bounces == 0: trace_ray_internal returns BLACK without a query
                 st3(a.L, p, mk3(0.f, 0.f, 0.f));
@@ -353,16 +355,17 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                     st3(a.L, p, fold_levels(a, p, depth, env, c));
                 } else {
                     float w = 1.f;
-                    float pb = a.pdf[p];
+                    const f32x4 Ap = a.A[p];
+                    float pb = Ap.w;
                     if ((r.flags & VR_RENDER_ENV_IS) && pb > 0.f && sv.env_kind == VR_ENV_HDRI) {
                         float pe = env_pdf_dir(sv, d);
                         w = (pb * pb) / (pb * pb + pe * pe);
                     }
-                    vf3 L = ld3(a.L, p), A = ld3(a.A, p);
+                    vf3 L = ld3(a.L, p), A = mk3(Ap.x, Ap.y, Ap.z);
                     st3(a.L, p, L + mulv(A, env) * w);
                 }
             } else {
-                HitRec hit = make_hit(sv, o, d, prim, a.hit_t[p], a.hit_u[p], a.hit_v[p]);
+                HitRec hit = make_hit(sv, o, d, prim, u2f(hw.y), u2f(hw.z), u2f(hw.w));
                 GpuMaterial m = sv.materials[hit.material];
                 textured = m.albedo_tex >= 0 || m.normal_tex >= 0;
                 if (!ext) {
@@ -388,10 +391,11 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                         }
                     }
                 } else {
-                    vf3 A = ld3(a.A, p), L = ld3(a.L, p);
+                    const f32x4 Ap = a.A[p];
+                    vf3 A = mk3(Ap.x, Ap.y, Ap.z), L = ld3(a.L, p);
                     const bool train_path =
                         CACHE && r.cmode == kCacheOn &&
-                        train_hash(a.path_pix[p], a.path_smp[p], r.request, r.frame) < r.train_threshold;
+                        train_hash(pix, smp, r.request, r.frame) < r.train_threshold;
                     const bool query = CACHE && r.cmode == kCacheOn && !train_path && depth >= r.cache_depth &&
                                        cache_roughness(m) >= r.query_roughness;
                     // a Lambertian's textures, read once for the record, next-event
@@ -429,7 +433,7 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                                 float pb = cw / kPi;
                                 float w = (pe * pe) / (pe * pe + pb * pb);
                                 vf3 contrib = mulv(mulv(A, ls.albedo), env_lookup(sv, wi)) * (pb * w / pe);
-                                st3(a.sh_o, p, hit.point);
+                                st3(a.ray_o, p, hit.point);
                                 st3(a.sh_d, p, wi);
                                 st3(a.sh_c, p, contrib);
                                 shadow = true;
@@ -450,9 +454,8 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
                                 else A = A / q;
                             }
                             if (alive) {
-                                st3(a.A, p, A);
-                                a.pdf[p] = pb;
-                                st3(a.ray_o, p, hit.point);
+                                a.A[p] = f32x4{A.x, A.y, A.z, pb};
+                                if (!shadow) st3(a.ray_o, p, hit.point);
                                 st3(a.ray_d, p, sc.dir);
                                 cont = true;
                             }
@@ -646,17 +649,16 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 size_t scratch_bytes(uint32_t cap, uint32_t att_levels, bool ext) {
     size_t b = 0;
     auto add = [&](size_t bytes) { b += align256(bytes); };
-    for (int k = 0; k < 3; ++k) add(4ull * cap);  // path req/pix/sample
+    add(12ull * cap);                              // path request/pixel/sample
     add(12ull * cap);                              // ray_o
     add(12ull * cap);                              // ray_d
-    for (int k = 0; k < 4; ++k) add(4ull * cap);  // hit prim/t/u/v
+    add(16ull * cap);                              // hit prim/t/u/v
     add(4ull * cap);                               // rng
     if (att_levels) add(12ull * cap * att_levels); // attenuation stack
     add(12ull * cap);                              // L
     if (ext) {
-        add(12ull * cap);                          // A
-        add(4ull * cap);                           // pdf
-        for (int k = 0; k < 3; ++k) add(12ull * cap);  // shadow o/d/c
+        add(16ull * cap);                          // A, pdf
+        for (int k = 0; k < 2; ++k) add(12ull * cap);  // shadow d/c
         add(1ull * cap);                           // shadow hit
         add(4ull * cap);                           // shadow queue
     }
@@ -987,22 +989,15 @@ static int enqueue_batch(vr_ctx* ctx, hipStream_t st) {
         a.reqs = R.d_reqs;
         a.cap = cap;
         char* cur = (char*)R.scratch;
-        a.path_req = carve<uint32_t>(cur, cap);
-        a.path_pix = carve<uint32_t>(cur, cap);
-        a.path_smp = carve<uint32_t>(cur, cap);
+        a.path_id = carve<uint32_t>(cur, 3ull * cap);
         a.ray_o = carve<float>(cur, 3ull * cap);
         a.ray_d = carve<float>(cur, 3ull * cap);
-        a.hit_prim = carve<uint32_t>(cur, cap);
-        a.hit_t = carve<float>(cur, cap);
-        a.hit_u = carve<float>(cur, cap);
-        a.hit_v = carve<float>(cur, cap);
+        a.hit = carve<u32x4>(cur, cap);
         a.rng_n = carve<uint32_t>(cur, cap);
         a.att = g.att_levels ? carve<float>(cur, 3ull * cap * g.att_levels) : nullptr;
         a.L = carve<float>(cur, 3ull * cap);
         if (g.any_ext) {
-            a.A = carve<float>(cur, 3ull * cap);
-            a.pdf = carve<float>(cur, cap);
-            a.sh_o = carve<float>(cur, 3ull * cap);
+            a.A = carve<f32x4>(cur, cap);
             a.sh_d = carve<float>(cur, 3ull * cap);
             a.sh_c = carve<float>(cur, 3ull * cap);
             a.sh_hit = carve<uint8_t>(cur, cap);
@@ -1041,10 +1036,7 @@ static int enqueue_batch(vr_ctx* ctx, hipStream_t st) {
                     j.tmin = 0.00001f;  // SceneAcceleration::hit (scene.rs:183)
                     j.any = false;
                     j.engine = (int)g.engine;
-                    j.prim = a.hit_prim;
-                    j.t = a.hit_t;
-                    j.u = a.hit_u;
-                    j.v = a.hit_v;
+                    j.rec = a.hit;
                     j.fallback_accum = R.stats_dev + 3;
                     int rc = launch_trace(s, j, st);
                     if (rc) return rc;
@@ -1061,7 +1053,7 @@ static int enqueue_batch(vr_ctx* ctx, hipStream_t st) {
                     hipLaunchKernelGGL(shade, dim3(grid_for(c.npaths, sb)), dim3(sb), 0, st, a, depth);
                     if (g.any_env_is) {
                         TraceJob sj;
-                        sj.o = a.sh_o;
+                        sj.o = a.ray_o;
                         sj.d = a.sh_d;
                         sj.n_max = c.npaths;
                         sj.queue = a.sh_queue;

@@ -55,6 +55,7 @@ struct TraceArgs {
     const uint32_t* count;  // optional: device-side item count (else n)
     float tmax;             // any-hit: hits at t >= tmax do not count
     int spill_cap;          // global spill entries per lane; a deeper stack hands the ray to the exact engine
+    u32x4* rec;             // optional: {prim, t, u, v} as one record (a path's hit)
 };
 
 // The kernel's arguments, for code outside the traversal loop (cold_scene).
@@ -63,6 +64,7 @@ __device__ __forceinline__ const TraceArgs& cold_args(const TraceArgs& a) {
 }
 
 __device__ __forceinline__ void write_out(const TraceArgs& a, uint32_t i, const HitOut& h) {
+    if (a.rec) a.rec[i] = u32x4{h.prim, f2u(h.t), f2u(h.u), f2u(h.v)};
     if (a.prim) a.prim[i] = h.prim;
     if (a.t) a.t[i] = h.t;
     if (a.u) a.u[i] = h.u;
@@ -805,7 +807,7 @@ struct TraceScratch {
 static int launch_trace_with(vr_scene* s, const TraceJob& j, const TraceScratch& sc, hipStream_t stream) {
     TraceArgs a{s->view, j.o, j.d, j.n_max, j.tmin, j.any ? 1 : 0, j.prim, j.t, j.u, j.v, j.hit,
                 sc.fb_list, sc.counters, sc.counters + kCtrFetch, sc.spill, sc.spill_lanes, j.queue, j.count, j.tmax,
-                sc.spill_cap};
+                sc.spill_cap, j.rec};
     const bool wt = j.engine == VR_ENGINE_WATERTIGHT;
     uint64_t* accum = j.engine != VR_ENGINE_REFERENCE ? j.fallback_accum : nullptr;
     if (j.engine != VR_ENGINE_REFERENCE) {
