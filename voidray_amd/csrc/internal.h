@@ -265,6 +265,9 @@ struct TraceJob {
     float *t = nullptr, *u = nullptr, *v = nullptr;
     uint8_t* hit = nullptr;
     u32x4* rec = nullptr;                // optional: {prim, t, u, v} per ray
+    // optional, [ray][3]: add_dst += add_src for the rays without a hit
+    const float* add_src = nullptr;
+    float* add_dst = nullptr;
     uint64_t* fallback_accum = nullptr;  // optional: += number of exact-engine rays
     bool timed = false;                  // record trace_ev[0..1] around the wide kernel
 };

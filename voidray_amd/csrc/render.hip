@@ -42,9 +42,9 @@ namespace vr {
 // thin them out, a small chunk leaves the traversal kernels' persistent waves
 // mostly idle.  On the 1080p x 64 spp terrain frame (132.7 M paths): 2^22
 // paths per chunk 394 ms, 2^24 215 ms, 2^26 (two chunks) 146 ms, 2^27 (one
-// chunk) 137 ms; about 121 B of path state per path with the extended
+// chunk) 137 ms; about 120 B of path state per path with the extended
 // estimator, 272 B with the reference estimator's 16-level attenuation stack:
-// 18 or 36 GB of the GPU's 288 GB at 2^27.  Scratch is sized by the largest
+// 16 or 36 GB of the GPU's 288 GB at 2^27.  Scratch is sized by the largest
 // chunk a call actually uses, so small frames allocate little.
 constexpr uint32_t kDefaultChunkPaths = 1u << 27;
 constexpr uint32_t kMaxChunkPaths = 1u << 27;
@@ -126,7 +126,6 @@ struct RenderArgs {
     float* L;    // [cap][3]
     f32x4* A;    // extended: throughput, pdf of the last diffuse scatter (0 = camera / specular)
     float *sh_d, *sh_c;
-    uint8_t* sh_hit;
     uint32_t* queue[2];
     uint32_t* sh_queue;
     uint32_t* cnt;
@@ -497,14 +496,6 @@ __global__ void k_shade(RenderArgs a, uint32_t depth) {
     }
 }
 
-__global__ void k_shadow_resolve(RenderArgs a, uint32_t depth) {
-    const uint32_t n = a.cnt[kCntShadow + depth];
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        uint32_t p = a.sh_queue[k];
-        if (a.sh_hit[p] == 0) st3(a.L, p, ld3(a.L, p) + ld3(a.sh_c, p));
-    }
-}
-
 // Cache queries of the chunk: L[path] += A * max(cache output, 0).
 __global__ void k_cache_apply(RenderArgs a) {
     const uint32_t n = min(*a.qr.count, a.qr.cap);
@@ -600,20 +591,29 @@ __global__ __launch_bounds__(kAccBlock) void k_accumulate(RenderArgs a) {
 
 // Adds one chunk's counters into the 64-bit statistics
 // [segments, samples, env misses, exact-engine rays, capped loops, textured hits, env IS samples].
-__global__ void k_stats_chunk(const uint32_t* cnt, uint64_t* stats, uint32_t npaths, uint32_t max_depth) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    uint64_t seg = max_depth ? npaths : 0;
-    for (uint32_t k = 1; k < max_depth; ++k) seg += cnt[kCntActive + k];
-    for (uint32_t k = 0; k < max_depth; ++k) seg += cnt[kCntShadow + k];
+// One wave, a counter per lane and step: by one thread, one after the other, the
+// about 220 reads of a chunk took 6.9 us; so 4.8, about what an empty launch takes.
+__global__ __launch_bounds__(64) void k_stats_chunk(const uint32_t* cnt, uint64_t* stats, uint32_t npaths,
+                                                    uint32_t max_depth) {
+    static_assert(kStatStripes == 64, "a lane per stripe");
+    const uint32_t lane = threadIdx.x;
+    uint64_t seg = lane == 0 && max_depth ? npaths : 0;
+    for (uint32_t k = lane; k < max_depth; k += 64u) {  // depth 0 is npaths
+        if (k) seg += cnt[kCntActive + k];
+        seg += cnt[kCntShadow + k];
+    }
+    const uint32_t* stripe = cnt + kCntStriped + lane * kStripeWords;
+    uint64_t miss = stripe[kStripeMiss], tex = stripe[kStripeTextured], env = stripe[kStripeEnvIS];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        seg += __shfl_xor(seg, off);
+        miss += __shfl_xor(miss, off);
+        tex += __shfl_xor(tex, off);
+        env += __shfl_xor(env, off);
+    }
+    if (lane != 0) return;
     stats[0] += seg;
     stats[1] += npaths;
-    uint64_t miss = 0, tex = 0, env = 0;
-    for (int s = 0; s < kStatStripes; ++s) {
-        const uint32_t* stripe = cnt + kCntStriped + s * kStripeWords;
-        miss += stripe[kStripeMiss];
-        tex += stripe[kStripeTextured];
-        env += stripe[kStripeEnvIS];
-    }
     stats[2] += miss;
     stats[4] += cnt[kCntCapped];
     stats[5] += tex;
@@ -659,7 +659,6 @@ size_t scratch_bytes(uint32_t cap, uint32_t att_levels, bool ext) {
     if (ext) {
         add(16ull * cap);                          // A, pdf
         for (int k = 0; k < 2; ++k) add(12ull * cap);  // shadow d/c
-        add(1ull * cap);                           // shadow hit
         add(4ull * cap);                           // shadow queue
     }
     add(4ull * cap);                               // queue 0
@@ -1000,7 +999,6 @@ static int enqueue_batch(vr_ctx* ctx, hipStream_t st) {
             a.A = carve<f32x4>(cur, cap);
             a.sh_d = carve<float>(cur, 3ull * cap);
             a.sh_c = carve<float>(cur, 3ull * cap);
-            a.sh_hit = carve<uint8_t>(cur, cap);
             a.sh_queue = carve<uint32_t>(cur, cap);
         }
         a.queue[0] = carve<uint32_t>(cur, cap);
@@ -1062,12 +1060,11 @@ static int enqueue_batch(vr_ctx* ctx, hipStream_t st) {
                         sj.tmax = kInf;
                         sj.any = true;
                         sj.engine = (int)g.engine;
-                        sj.hit = a.sh_hit;
+                        sj.add_src = a.sh_c;  // unoccluded: L += the sample's contribution
+                        sj.add_dst = a.L;
                         sj.fallback_accum = R.stats_dev + 3;
                         rc = launch_trace(s, sj, st);
                         if (rc) return rc;
-                        hipLaunchKernelGGL(k_shadow_resolve, dim3(grid_for(c.npaths, sb)), dim3(sb), 0, st, a,
-                                           depth);
                     }
                 }
                 if (g.any_cached) {

@@ -56,6 +56,8 @@ struct TraceArgs {
     float tmax;             // any-hit: hits at t >= tmax do not count
     int spill_cap;          // global spill entries per lane; a deeper stack hands the ray to the exact engine
     u32x4* rec;             // optional: {prim, t, u, v} as one record (a path's hit)
+    const float* add_src;   // optional, [ray][3]: a ray without a hit adds its entry to
+    float* add_dst;         // its entry here (a path's next-event radiance)
 };
 
 // The kernel's arguments, for code outside the traversal loop (cold_scene).
@@ -65,6 +67,14 @@ __device__ __forceinline__ const TraceArgs& cold_args(const TraceArgs& a) {
 
 __device__ __forceinline__ void write_out(const TraceArgs& a, uint32_t i, const HitOut& h) {
     if (a.rec) a.rec[i] = u32x4{h.prim, f2u(h.t), f2u(h.u), f2u(h.v)};
+    if (a.add_dst && h.prim == 0xFFFFFFFFu) {
+        const float* s = a.add_src + 3 * (size_t)i;
+        float* d = a.add_dst + 3 * (size_t)i;
+        const vf3 sum = mk3(d[0], d[1], d[2]) + mk3(s[0], s[1], s[2]);
+        d[0] = sum.x;
+        d[1] = sum.y;
+        d[2] = sum.z;
+    }
     if (a.prim) a.prim[i] = h.prim;
     if (a.t) a.t[i] = h.t;
     if (a.u) a.u[i] = h.u;
@@ -555,6 +565,14 @@ __global__ __launch_bounds__(kWave) void k_trace_exact_wave(TraceArgs a, const u
     // part in the exit count.  A block that leaves may read the count after
     // the reset, but then it reads 0 and leaves all the same: the reset only
     // happens once every taking-part block has read the count.
+    // (Without a ray, the usual case, there is no list to run and nobody to wait
+    // for: block 0 resets without the fences and the count.  64 rays: 31.6 -> 30.7 us.)
+    if (n == 0u) {
+        if (blockIdx.x != 0u) return;
+        if (lane == 0) ctr[kCtrLastFallbacks] = ctr[kCtrLastOverflow] = 0u;
+        if (lane < kFetchParts) ctr[kCtrFetch + lane * kFetchStride] = 0u;
+        return;
+    }
     const uint32_t parts = n < gridDim.x ? (n > 1u ? n : 1u) : gridDim.x;
     if (blockIdx.x >= parts) return;
     for (uint32_t j = blockIdx.x; j < n; j += gridDim.x) {
@@ -807,7 +825,7 @@ struct TraceScratch {
 static int launch_trace_with(vr_scene* s, const TraceJob& j, const TraceScratch& sc, hipStream_t stream) {
     TraceArgs a{s->view, j.o, j.d, j.n_max, j.tmin, j.any ? 1 : 0, j.prim, j.t, j.u, j.v, j.hit,
                 sc.fb_list, sc.counters, sc.counters + kCtrFetch, sc.spill, sc.spill_lanes, j.queue, j.count, j.tmax,
-                sc.spill_cap, j.rec};
+                sc.spill_cap, j.rec, j.add_src, j.add_dst};
     const bool wt = j.engine == VR_ENGINE_WATERTIGHT;
     uint64_t* accum = j.engine != VR_ENGINE_REFERENCE ? j.fallback_accum : nullptr;
     if (j.engine != VR_ENGINE_REFERENCE) {
