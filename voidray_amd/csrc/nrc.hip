@@ -42,7 +42,11 @@ namespace {
 
 constexpr float kInvPi = 0.31830988618379067f;
 constexpr float kInv2Pi = 0.15915494309189535f;
-constexpr int kWgradBlocks = 64;
+// Sample blocks of k_nrc_wgrad (and partials of k_nrc_reduce).  65,536 samples,
+// the whole gradient call: 64 blocks 440 us (each block's chain of loads is the
+// time), 128 415, 256 413 with twice the partials; eight mini-batches of 8,192 the
+// same with 32, 64 and 128.
+constexpr int kWgradBlocks = 128;
 constexpr int kFwdBlock = 256;
 
 // LDS copy of the weights with padded rows (bank-conflict-free 16-byte reads)
@@ -641,12 +645,23 @@ __global__ __launch_bounds__(256) void k_nrc_wgrad(const __bf16* xT, const __bf1
     }
 }
 
-__global__ void k_nrc_reduce(const float* part, uint32_t blocks, float* grad) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint32_t)kNrcParams) return;
+// Sums the blocks' partials (a multiple of 4), in a fixed order: a block of four
+// waves sums 64 parameters, a quarter of the partials each.  Bound by the
+// latency of its reads: one thread a parameter, 84 blocks in all, took 16.4 us,
+// this takes 4.7 (with twice the partials).
+__global__ __launch_bounds__(256) void k_nrc_reduce(const float* part, uint32_t blocks, float* grad) {
+    static_assert(kNrcParams % 64 == 0, "no remainder");
+    static_assert(kWgradBlocks % 4 == 0, "a quarter of the partials per wave");
+    __shared__ float sum[4][64];
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6, i = blockIdx.x * 64u + lane;
+    const uint32_t q = blocks / 4u;
+    const float* p = part + (size_t)w * q * kNrcParams + i;
     float s = 0.f;
-    for (uint32_t b = 0; b < blocks; ++b) s += part[(size_t)b * kNrcParams + i];
-    grad[i] = s;
+#pragma unroll 8
+    for (uint32_t b = 0; b < q; ++b) s += p[(size_t)b * kNrcParams];
+    sum[w][lane] = s;
+    __syncthreads();
+    if (w == 0) grad[i] = (sum[0][lane] + sum[1][lane]) + (sum[2][lane] + sum[3][lane]);
 }
 
 // All-FP32 debug path: one thread per sample, weights and grid from the FP32
@@ -978,7 +993,7 @@ int nrc_train_step(vr_cache* c, uint32_t n, const uint32_t* d_n, const float* po
             hipLaunchKernelGGL(k_nrc_wgrad, dim3(kWgradBlocks, 5), dim3(256), 0, st, (const __bf16*)c->xT,
                                (const __bf16*)c->hT, (const __bf16*)c->dT, c->train_cap, d_n, n, part, parts,
                                c->part);
-            hipLaunchKernelGGL(k_nrc_reduce, dim3((kNrcParams + 255) / 256), dim3(256), 0, st, (const float*)c->part,
+            hipLaunchKernelGGL(k_nrc_reduce, dim3(kNrcParams / 64), dim3(256), 0, st, (const float*)c->part,
                                (uint32_t)kWgradBlocks, c->w_grad);
         }
     }
