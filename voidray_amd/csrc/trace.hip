@@ -501,23 +501,25 @@ template <>
 __global__ __launch_bounds__(kWave, 7) void k_trace_persist<true, true, false>(TraceArgs a) {
     trace_persist<true, true, false>(a);
 }
-// scenes with instances (the instance bookkeeping needs more registers, about
-// 110: held to 5 to 7 waves per SIMD the kernels spill, and a 960 x 540 x 4
-// frame of 200 instances took 11.1 ms instead of 6.9)
+// scenes with instances (the instance bookkeeping needs more registers): 5 waves
+// per SIMD, 96 VGPRs, 4 of the watertight kernels' spilled.  Frames of 200
+// instances with 4, 5 and 6 waves: 960 x 540 x 4 5.65, 5.51 and 5.64 ms
+// (watertight 5.73, 5.64, 6.28), 1080p x 16 37.2, 34.9 and 34.6 ms (37.6, 35.7,
+// 41.5); at 7 dozens of registers spill.
 template <>
-__global__ __launch_bounds__(kWave, 4) void k_trace_persist<false, false, true>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 5) void k_trace_persist<false, false, true>(TraceArgs a) {
     trace_persist<false, false, true>(a);
 }
 template <>
-__global__ __launch_bounds__(kWave, 4) void k_trace_persist<true, false, true>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 5) void k_trace_persist<true, false, true>(TraceArgs a) {
     trace_persist<true, false, true>(a);
 }
 template <>
-__global__ __launch_bounds__(kWave, 4) void k_trace_persist<false, true, true>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 5) void k_trace_persist<false, true, true>(TraceArgs a) {
     trace_persist<false, true, true>(a);
 }
 template <>
-__global__ __launch_bounds__(kWave, 4) void k_trace_persist<true, true, true>(TraceArgs a) {
+__global__ __launch_bounds__(kWave, 5) void k_trace_persist<true, true, true>(TraceArgs a) {
     trace_persist<true, true, true>(a);
 }
 
