@@ -284,8 +284,8 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0                               # MI355X dense BF16
 def _cache_roofline(ctx, torch, stream, lo, hi, n_infer=1 << 20, n_train=1 << 16, reps=10):
     """MFMA roofline of the learned cache's kernels, timed live with HIP events
     on the stream they run on: inference (one k_nrc_infer launch over n_infer
-    queries) and one training step over n_train samples (k_nrc_train with its
-    grid-gradient atomics, k_nrc_wgrad, the reduction and Adam).  Queries:
+    queries) and one training step over n_train samples (k_nrc_train,
+    k_nrc_scatter, k_nrc_wgrad, the reduction and Adam).  Queries:
     positions uniform in the scene box, random unit directions and normals,
     roughness U(0, 1); training targets U(0, 1)."""
     from voidray_amd.device import RadianceCache
@@ -767,7 +767,7 @@ def main():
         "dtype": "f32",
         "data": "synthetic",
         "config": {"workload": "traversal microbench", "triangles": args.tris, "rays": n,
-                   "rays_mix": "1/2 coherent 2048^2 pinhole, 1/2 incoherent", "bvh": "SAH + spatial splits, 4-wide, 8-bit quantised",
+                   "rays_mix": "1/2 coherent 2048^2 pinhole, 1/2 incoherent", "bvh": "SAH + spatial splits, 8-wide, 8-bit quantised",
                    "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": pmc.get("hbm_bytes_per_launch"),

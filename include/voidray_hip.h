@@ -234,7 +234,7 @@ int vr_scene_get_stats(const vr_scene* scene, vr_scene_stats* out);
  * records per call, a few microseconds; off by default). */
 #define VR_TRACE_TIMING 0x100
 /* traversal engines */
-#define VR_ENGINE_WIDE 0      /* quantised BVH4 + robust-winner check + exact fallback */
+#define VR_ENGINE_WIDE 0      /* quantised BVH8 + robust-winner check + exact fallback */
 #define VR_ENGINE_REFERENCE 1 /* flattened reference trees, both children, no pruning  */
 /* The wide BVH with the watertight ray/triangle test (Woop, Benthin & Wald,
  * JCGT 2013) in place of Moller-Trumbore: no ray slips between the triangles

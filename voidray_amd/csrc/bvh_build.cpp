@@ -134,7 +134,7 @@ void build_reference_tree(const std::vector<Box3>& bounds, std::vector<RefNode>&
 }
 
 // ---------------------------------------------------------------------------
-// SAH binary BVH -> 4-wide quantised BVH
+// SAH binary BVH -> 8-wide quantised BVH
 // ---------------------------------------------------------------------------
 
 namespace {

@@ -317,7 +317,7 @@ int build_host_scene(const vr_scene_desc* d, HostScene& H) {
     }
     auto t_ref1 = clk::now();
 
-    // ---- fast structure: triangle records + SAH quantised BVH4 ------------
+    // ---- fast structure: triangle records + SAH quantised BVH8 ------------
     std::vector<TriRec> recs;
     recs.reserve(T);
     std::vector<PrimRec>& prims = H.prims;
