@@ -55,9 +55,9 @@ constexpr size_t kDefaultScratchBudget = 48ull << 30;
 constexpr uint32_t kMaxBouncesLimit = 64;
 // Most threads a grid-stride kernel over a chunk launches: one round of the
 // shading kernel's resident waves (256 CUs x 16 waves at its 128 VGPRs = 4,096
-// waves), e.g. 256 blocks of 1,024 threads.  With blocks of 256, 1,024 blocks
-// beat 2,048 on the render legs (cornell 5%, the 1080p frames 0.5-0.7%), and
-// 768 or 512 left CUs idle (up to 11% slower).
+// waves), e.g. 512 blocks of 512 threads.  Twice as many threads: cornell 4%,
+// the 719p x 8 reference frame 5% slower (the appends mix paths from farther
+// apart); a quarter more: 13% and 7%, the last round of blocks part empty.
 constexpr uint32_t kShadeThreads = 4096u * 64u;
 
 // Blocks of a grid-stride kernel over at most n items.
@@ -768,9 +768,11 @@ static int plan_batch(vr_ctx* ctx, const vr_request* items, uint32_t n, const vr
     RenderState& R = *ctx->render;
     uint32_t chunk_paths = tune.chunk_paths ? tune.chunk_paths : kDefaultChunkPaths;
     if (chunk_paths > kMaxChunkPaths) return fail(VR_ERR_INVALID, "chunk_paths above 2^27");
-    // 1,024 threads: on the render legs 4% faster than 256 on cornell, 0.6-1.2%
-    // on the 1080p frames (fewer blocks, one queue atomic per block), 128 slower
-    uint32_t block = tune.block ? tune.block : 1024;
+    // 512 threads: the shading kernel's appends join 8 waves at each barrier.  With
+    // 1,024 and 256: cornell 2.68 and 2.74 ms instead of 2.62, the 719p x 8
+    // reference frame 6.82 and 6.82 instead of 6.76, 16 mixed requests 50.4 and
+    // 49.8 instead of 49.9, a 161 x 97 preview 359 and 335 us instead of 346.
+    uint32_t block = tune.block ? tune.block : 512;
     if (block % 64 != 0 || block > 1024) return fail(VR_ERR_INVALID, "block must be a multiple of 64 up to 1024");
     drop_graph(R);
     R.reqs.clear();
